@@ -26,6 +26,7 @@ struct LaunchCfg {
   int t_block = 1;  // fused time steps per pass
   int variant = 0;  // sweep tile variant (0 = default tile)
   int xcd_order = 1;  // renumber workgroups per XCD
+  int ftile = 0;      // output tile of the fused pass, where its depth has several (fused_tiles)
 };
 
 int num_tile_variants(int kid, int dtype);
@@ -47,9 +48,15 @@ extern thread_local int *g_fused_tile_probe;
 // Output tile of the fused pass of depth tl that tblock_pass would launch for P and lc;
 // false where there is no such pass.
 bool fused_tile(const Problem &P, int tl, const LaunchCfg &lc, int *tx, int *ty);
+// Output tiles that the fused pass of depth tl has (LaunchCfg::ftile).
+int fused_tiles(const Problem &P, int tl);
 hipError_t tblock_pass(const Problem &P, int tl, const void *X, const void *Y, void *ZO, void *ZN, const void *src,
                        long long src_idx, const LaunchCfg &lc, hipStream_t st);
 int tb_depths(int kid, int dtype, int *out, int max);
+// tl kernel-5 steps per pass (Y -> Z), and the output tiles of that depth.
+hipError_t k5_pass(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+                   const LaunchCfg &lc, hipStream_t st);
+int k5_tiles(const Problem &P, int tl);
 // tl kernel-1 steps per pass: Y -> Z.
 hipError_t jacobi_tb_pass(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
                           const LaunchCfg &lc, hipStream_t st);

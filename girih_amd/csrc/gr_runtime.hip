@@ -167,11 +167,11 @@ using namespace gr;
 
 // What a captured step sequence depends on besides the (fixed) field allocations.
 struct GraphKey {
-  int napply, parity, lu0, lu1, variant, zchunk, t_block, xcd_order, fuse;
+  int napply, parity, lu0, lu1, variant, zchunk, t_block, xcd_order, ftile, fuse;
   long long napplied;  // -1 unless a source is active (its pointers are baked into the graph)
   bool operator==(const GraphKey &o) const {
     return napply == o.napply && parity == o.parity && lu0 == o.lu0 && lu1 == o.lu1 && variant == o.variant &&
-           zchunk == o.zchunk && t_block == o.t_block && xcd_order == o.xcd_order && fuse == o.fuse &&
+           zchunk == o.zchunk && t_block == o.t_block && xcd_order == o.xcd_order && ftile == o.ftile && fuse == o.fuse &&
            napplied == o.napplied;
   }
 };
@@ -530,7 +530,7 @@ extern "C" int gr_step(gr_handle *h, int napply) {
   }
   // graph mode: replay the launch sequence of an identical earlier call
   GraphKey key{napply, h->parity, h->lu[0], h->lu[1], h->lc.variant, h->lc.zchunk, h->lc.t_block, h->lc.xcd_order,
-               fuse ? 1 : 0, -1};
+               h->lc.ftile, fuse ? 1 : 0, -1};
   if (h->src && h->napplied < h->nsrc) key.napplied = h->napplied;  // source pointers are baked in
   if (h->use_graph && napply > 0) {
     if (!(h->gexec && h->gkey == key)) {
@@ -703,6 +703,9 @@ extern "C" int gr_set_config(gr_handle *h, int variant, int zchunk, int t_block)
     }
     h->lc.t_block = t_block;
   }
+  // the fused pass's output tile goes by the tile variant where its depth has that many
+  if (variant >= 0 || t_block >= 1)
+    h->lc.ftile = h->lc.variant < fused_tiles(h->P, h->lc.t_block) ? h->lc.variant : 0;
   return GR_OK;
 }
 
@@ -748,6 +751,8 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
   h->spares_synced = true;  // copies of the fields: same halo
   void *a = field_base(h, h->fbuf[sp[0]]), *b = field_base(h, h->fbuf[sp[1]]);
   const int nz = P.nz;
+  int ncu = 0;
+  HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device));
   std::vector<int> zchunks = {0};
   for (int zc : {512, 256, 128, 64, 32})
     if (zc < nz) zchunks.push_back(zc);
@@ -783,8 +788,10 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
   };
   // stage 1: tile variant x workgroup order at each z-chunk size of a coarse set;
   // stage 2: all z-chunk sizes and orders for the best variant
-  for (int var = 0; var < num_tile_variants(P.kernel, P.dtype); ++var)
-    for (int order = 0; order < 3; ++order)
+  // (a variant whose plain order is far from the best so far skips the other orders)
+  for (int var = 0; var < num_tile_variants(P.kernel, P.dtype); ++var) {
+    float var_ms = 1e30f;
+    for (int order = 0; order < 3 && !(order > 0 && var_ms > 1.4f * best_ms); ++order)
       for (int zc : {0, std::min(128, nz)}) {
         LaunchCfg lc = h->lc;
         lc.variant = var;
@@ -792,7 +799,9 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
         lc.zchunk = zc;
         lc.t_block = 1;
         if ((rc = trial(lc))) return rc;
+        var_ms = std::min(var_ms, tried.back().first);
       }
+  }
   {
     const LaunchCfg base = best_lc;
     for (int order = 0; order < 3; ++order)
@@ -844,9 +853,30 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
       if (!ok) continue;
       const int tl = depths[i];
       const int npass = (steps + tl - 1) / tl;
-      for (int zc : zchunks)
-      for (int order = 0; order < 3; ++order) {  // XCD-contiguous orders keep the per-level re-reads in one L2
+      for (int ft = 0; ft < fused_tiles(P, tl); ++ft) {
+      std::vector<int> zcs;
+      {  // first the chunks that make the workgroups one to four full rounds of the GPU's CUs
         LaunchCfg lc = best_lc;
+        lc.ftile = ft;
+        int tx = 0, ty = 0;
+        if (fused_tile(P, tl, lc, &tx, &ty)) {
+          const int ntile = ((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty);
+          for (int r = 1; r <= 4; ++r) {
+            const int nzc = r * ncu / ntile;
+            const int zc = nzc > 0 ? (nz + nzc - 1) / nzc : 0;
+            if (zc >= 2 * tl && zc < nz && std::find(zcs.begin(), zcs.end(), zc) == zcs.end()) zcs.push_back(zc);
+          }
+        }
+        for (int zc : zchunks)
+          if (std::find(zcs.begin(), zcs.end(), zc) == zcs.end()) zcs.push_back(zc);
+      }
+      // (a tile whose first chunk lengths are far from the best so far skips the others)
+      float tile_ms = 1e30f;
+      for (size_t iz = 0; iz < zcs.size() && !(iz >= 2 && tile_ms > 1.4f * best_ms); ++iz)
+      for (int order = 0; order < 3; ++order) {  // XCD-contiguous orders keep the margins' re-reads in one L2
+        const int zc = zcs[iz];
+        LaunchCfg lc = best_lc;
+        lc.ftile = ft;
         lc.t_block = tl;
         lc.zchunk = zc;
         lc.xcd_order = order;
@@ -864,10 +894,12 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
         const float per_step = ms * steps / (float)(npass * tl);  // comparable with the sweep trials
+        tile_ms = std::min(tile_ms, per_step);
         if (per_step < best_ms) {
           best_ms = per_step;
           best_lc = lc;
         }
+      }
       }
     }
   }

@@ -1,0 +1,73 @@
+// gr_star7_k5.hip -- dispatch of kernel 5's temporally blocked passes (gr_star7.hpp).
+#include <hip/hip_runtime.h>
+#include <hip/hip_bf16.h>
+
+#include "../../include/girih_gpu.h"
+#include "gr_internal.hpp"
+#include "gr_star7_launch.hpp"
+
+namespace gr {
+
+// Tiles per precision and depth; `tile` 0 is the default, the autotuner tries them all.
+// What bounds a pass is the memory fabric: it moves the coefficients and the field of
+// the computed region (tile + margins, less what neighbouring tiles find in the L2) once
+// per TL steps.  So the tile is as large as the registers allow at one workgroup per
+// CU: TL x 7 coefficient words, 3 x TL queue words and the next plane's 8 per cell.
+// Lanes own 4 cells in x (FP32, bf16) or 2 (FP64): fewer instructions per cell, and a
+// 256-VGPR budget at 7-8 waves per CU.  512^3, one box, 4 passes, GLUP/s, against the
+// pass with one barrier per level and coefficients loaded where level 1 uses them:
+//   FP32 depth 4: 64 x 16, 448 lanes x 4 cells 459 (2.75 GB/pass HBM write+fetch 5.9 GB,
+//     5.1 TB/s), 832 lanes x 2 cells 360 (spills); before 284
+//   bf16 depth 4: 128 x 16, 768 lanes x 4 cells 714; 64 x 32, 704 lanes x 4 668; 64 x 16,
+//     832 lanes x 2 636; before 388.  Depth 6, 64 x 16, 1024 lanes x 2: 703; before 322
+//   FP64 depth 4: 64 x 8, 512 lanes x 2 cells 245 (6.6 TB/s); 1024 lanes x 1 187
+//     (spills), 32 x 18 210; before 128
+//   depth 2: FP32 64 x 32 245, 128 x 16 262 (before 217); bf16 64 x 32 382 (258);
+//     FP64 64 x 16 138 (104)
+template <typename T, typename C>
+static hipError_t k5_dispatch(int tl, int tile, const S7Args<T, C> &a, hipStream_t st) {
+  constexpr bool B16 = std::is_same<C, __hip_bfloat16>::value;
+  if constexpr (B16) {
+    if (tl == 2) return launch_s7<T, C, 5, 2, 64, 32, 640, 4, false>(a, st);
+    if (tl == 4) {
+      if (tile == 1) return launch_s7<T, C, 5, 4, 128, 16, 768, 4, false>(a, st);
+      if (tile == 2) return launch_s7<T, C, 5, 4, 64, 16, 832, 2, false>(a, st);
+      return launch_s7<T, C, 5, 4, 64, 32, 704, 4, false>(a, st);
+    }
+    if (tl == 6) return launch_s7<T, C, 5, 6, 64, 16, 1024, 2, false>(a, st);
+  } else if constexpr (sizeof(T) == 4) {
+    if (tl == 2) {
+      if (tile == 1) return launch_s7<T, C, 5, 2, 128, 16, 704, 4, false>(a, st);
+      return launch_s7<T, C, 5, 2, 64, 32, 640, 2, false>(a, st);
+    }
+    if (tl == 4) return launch_s7<T, C, 5, 4, 64, 16, 448, 4, false>(a, st);
+  } else {
+    if (tl == 2) return launch_s7<T, C, 5, 2, 64, 16, 704, 2, false>(a, st);
+    if (tl == 4) return launch_s7<T, C, 5, 4, 64, 8, 512, 2, false>(a, st);
+  }
+  return hipErrorInvalidValue;
+}
+
+int k5_tiles(const Problem &P, int tl) {
+  if (P.flags & GR_COEF_BF16) return tl == 4 ? 3 : 1;
+  return P.dtype == GR_F32 && tl == 2 ? 2 : 1;
+}
+
+template <typename T, typename C>
+static hipError_t k5_pass_t(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+                            const LaunchCfg &lc, hipStream_t st) {
+  S7Args<T, C> a = s7_args<T, C>(P, Y, Z, src, src_idx, lc);
+  a.coef = (const C *)P.coef - P.xoff;  // addressed with the fields' element index
+  a.cstride = P.field_elems;
+  return k5_dispatch<T, C>(tl, lc.ftile, a, st);
+}
+
+// One pass of tl kernel-5 steps: Y -> Z.
+hipError_t k5_pass(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+                   const LaunchCfg &lc, hipStream_t st) {
+  if (P.dtype == GR_F64) return k5_pass_t<double, double>(P, tl, Y, Z, src, src_idx, lc, st);
+  if (P.flags & GR_COEF_BF16) return k5_pass_t<float, __hip_bfloat16>(P, tl, Y, Z, src, src_idx, lc, st);
+  return k5_pass_t<float, float>(P, tl, Y, Z, src, src_idx, lc, st);
+}
+
+}  // namespace gr

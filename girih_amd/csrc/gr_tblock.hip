@@ -22,11 +22,13 @@
 // Boundary cells (girih's halo, never updated) keep their input value at every
 // level; the host enables this path only when U1 and U2 hold the same halo.
 //
-// This kernel serves kernel 5 (seven coefficient arrays, FP64, FP32 or bf16-stored):
-// level t = f(level t-1), input Y, output ZN.  Kernel 1 has a leaner pass in gr_fused1.hip and kernel 0
-// (second order in time) a two-step pass in gr_wave2.hip.
+// This kernel serves kernel 5 (seven coefficient arrays, FP64 or FP32) at depth 6, where
+// six planes of coefficients do not fit the registers and every level reads its own
+// again: level t = f(level t-1), input Y, output ZN.  The other depths of kernel 5 keep
+// them on chip (gr_star7.hpp; at depth 6 that form, reading them at every level, ran 121
+// against 183-198 GLUP/s here in FP32 at 512^3).  Kernel 1 has a leaner pass in
+// gr_fused1.hip and kernel 0 (second order in time) a two-step pass in gr_wave2.hip.
 #include <hip/hip_runtime.h>
-#include <hip/hip_bf16.h>
 
 #include "../../include/girih_gpu.h"
 #include "gr_internal.hpp"
@@ -34,12 +36,11 @@
 
 namespace gr {
 
-// C: storage type of the coefficient arrays (T, or bf16 widened exactly to FP32)
-template <typename T, typename C>
+template <typename T>
 struct TbArgs {
   const T *Y;   // level 0
   T *ZN;        // level TL
-  const C *coef;
+  const T *coef;
   long long cstride;
   long long sy, sz;
   int nx, ny, nz;  // interior; boxes are [R, n+R)
@@ -49,11 +50,8 @@ struct TbArgs {
   int src_k, src_off;
 };
 
-// CP: level t+1 takes plane p's coefficients from level t one step earlier (same lane
-// and column) instead of re-reading them; costs TL x 7 registers per column, or TL x 4
-// with bf16 coefficients, which are handed on as stored, two to a register.
-template <typename T, typename C, int KID, int NT, int TXO, int TYO, int TL, bool CP>
-__global__ __launch_bounds__(NT) void tb_kernel(const TbArgs<T, C> a) {
+template <typename T, int KID, int NT, int TXO, int TYO, int TL>
+__global__ __launch_bounds__(NT) void tb_kernel(const TbArgs<T> a) {
   static_assert(KID == 5, "kernel 5 only");
   constexpr int R = kradius(KID);
   constexpr int Q = 2 * R + 1;
@@ -155,28 +153,11 @@ __global__ __launch_bounds__(NT) void tb_kernel(const TbArgs<T, C> a) {
   };
   fetch0(kfirst);
 
-  // cs[t-1][j]: the coefficients level t uses in this step.  Level t+1 is live at
-  // (step k0+1, column j) only where level t was live at (k0, j) on the same plane p =
-  // k0 - t: level regions shrink with t and level t+1 starts R planes later.  bf16
-  // coefficients are handed on as stored, two to a register (PK).
-  constexpr bool PK = CP && std::is_same<C, __hip_bfloat16>::value;
-  constexpr int CW = PK ? 4 : 7;  // registers per column and level
-  using CS = typename std::conditional<PK, unsigned, T>::type;
-  CS cs[CP ? TL : 1][NCOL][CW];
-
   for (int kb = kfirst; kb < klast; kb += Q) {
 #pragma unroll
     for (int ph = 0; ph < Q; ++ph) {
       const int k0 = kb + ph;
       if (k0 >= klast) break;
-      if constexpr (CP) {
-#pragma unroll
-        for (int t = TL - 1; t >= 1; --t)
-#pragma unroll
-          for (int j = 0; j < NCOL; ++j)
-#pragma unroll
-            for (int m = 0; m < CW; ++m) cs[t][j][m] = cs[t - 1][j][m];
-      }
       // slot of plane p: ((p mod Q) + Q) mod Q; k0 - kfirst = kb - kfirst + ph and
       // (kb - kfirst) is a multiple of Q, so plane k0 - R*t sits in slot
       // (ph - R*t) mod Q relative to kfirst's slot 0.
@@ -226,37 +207,10 @@ __global__ __launch_bounds__(NT) void tb_kernel(const TbArgs<T, C> a) {
               for (int d = -R; d <= R; ++d) zq[R + d] = zn(d);
               const T v0 = zq[R];
               {  // stencils.c:193-201; coefficients re-read by every level stay cached
-                const C *cp = a.coef + (long long)p * a.sz + off[j] / sizeof(T);
-                if constexpr (PK) {  // the bits of a bf16 value are the top half of its FP32 value
-                  if (t == 1) {
-                    const unsigned short *cb = reinterpret_cast<const unsigned short *>(cp);
-                    unsigned short h[7];
-#pragma unroll
-                    for (int m = 0; m < 7; ++m) h[m] = cb[m * a.cstride];
-#pragma unroll
-                    for (int w = 0; w < 3; ++w) cs[0][j][w] = (unsigned)h[2 * w] | ((unsigned)h[2 * w + 1] << 16);
-                    cs[0][j][3] = h[6];
-                  }
-                  const unsigned *w = cs[t - 1][j];
-                  T c[7];
-#pragma unroll
-                  for (int m = 0; m < 7; ++m)
-                    c[m] = __uint_as_float((m & 1) ? (w[m >> 1] & 0xffff0000u) : (w[m >> 1] << 16));
-                  out = c[0] * v0 + c[1] * xn(-1) + c[2] * xn(1) + c[3] * yn(-1) + c[4] * yn(1) + c[5] * zq[0] +
-                        c[6] * zq[2];
-                } else if constexpr (CP) {
-                  if (t == 1) {
-#pragma unroll
-                    for (int m = 0; m < 7; ++m) cs[0][j][m] = ld_coef<T, C, false>(cp + m * a.cstride);
-                  }
-                  const T *c = cs[CP ? t - 1 : 0][j];
-                  out = c[0] * v0 + c[1] * xn(-1) + c[2] * xn(1) + c[3] * yn(-1) + c[4] * yn(1) + c[5] * zq[0] +
-                        c[6] * zq[2];
-                } else {
-                  auto cf = [&](int m) { return ld_coef<T, C, false>(cp + m * a.cstride); };
-                  out = cf(0) * v0 + cf(1) * xn(-1) + cf(2) * xn(1) + cf(3) * yn(-1) + cf(4) * yn(1) +
-                        cf(5) * zq[0] + cf(6) * zq[2];
-                }
+                const T *cp = a.coef + (long long)p * a.sz + off[j] / sizeof(T);
+                auto cf = [&](int m) { return cp[m * a.cstride]; };
+                out = cf(0) * v0 + cf(1) * xn(-1) + cf(2) * xn(1) + cf(3) * yn(-1) + cf(4) * yn(1) +
+                      cf(5) * zq[0] + cf(6) * zq[2];
               }
               if (a.src_k >= 0 && p == a.src_k && off[j] == (unsigned)a.src_off * (unsigned)sizeof(T)) out = out + a.src[t - 1];
             } else {
@@ -292,19 +246,19 @@ __global__ __launch_bounds__(NT) void tb_kernel(const TbArgs<T, C> a) {
   }
 }
 
-template <typename T, typename C, int KID, int NT, int TXO, int TYO, int TL, bool CP = false>
-static hipError_t launch_tb(const TbArgs<T, C> &a0, hipStream_t st) {
+template <typename T, int KID, int NT, int TXO, int TYO, int TL>
+static hipError_t launch_tb(const TbArgs<T> &a0, hipStream_t st) {
   if (g_fused_tile_probe) {
     g_fused_tile_probe[0] = TXO;
     g_fused_tile_probe[1] = TYO;
     return hipSuccess;
   }
-  TbArgs<T, C> a = a0;
+  TbArgs<T> a = a0;
   a.tiles_x = (a.nx + TXO - 1) / TXO;
   a.tiles_y = (a.ny + TYO - 1) / TYO;
   a.zchunk = (a.zchunk <= 0 || a.zchunk > a.nz) ? a.nz : a.zchunk;
   a.nzc = (a.nz + a.zchunk - 1) / a.zchunk;
-  hipLaunchKernelGGL((tb_kernel<T, C, KID, NT, TXO, TYO, TL, CP>), dim3(a.tiles_x * a.tiles_y * a.nzc), dim3(NT), 0, st, a);
+  hipLaunchKernelGGL((tb_kernel<T, KID, NT, TXO, TYO, TL>), dim3(a.tiles_x * a.tiles_y * a.nzc), dim3(NT), 0, st, a);
   return hipGetLastError();
 }
 
@@ -317,7 +271,7 @@ int tb_depths(int kid, int dtype, int *out, int max) {
   (void)dtype;
   if (kid == 1) {  // gr_fused1.hip
     for (int d = 2; d <= 6; ++d) add(d);
-  } else if (kid == 5) {  // tb_kernel
+  } else if (kid == 5) {  // gr_star7_k5.hip; depth 6 without bf16 coefficients: tb_kernel
     add(2);
     add(4);
     add(6);
@@ -327,52 +281,14 @@ int tb_depths(int kid, int dtype, int *out, int max) {
   return n;
 }
 
-// Tiles per kernel and precision, sized so the per-lane queues (levels x columns
-// x (2R+1) words) and the coefficient hand-off stay in registers without spilling.
-template <typename T, typename C>
-static hipError_t tb_dispatch(int kid, int tl, const TbArgs<T, C> &a, hipStream_t st) {
-  constexpr bool F32 = std::is_same<T, float>::value;
-  constexpr bool B16 = std::is_same<C, __hip_bfloat16>::value;
-  if (kid == 5) {
-    // depth 2, coefficient hand-off. FP32: 896 lanes give 3 columns per lane (66 x 34
-    // level-1 cells), 86 VGPRs and 5 waves per SIMD, against 5 columns, 139 VGPRs and
-    // 3 waves with 512 lanes.  FP64: 640 lanes give 2 columns per lane (66 x 18
-    // level-1 cells), 112 VGPRs and 4 waves per SIMD, against 3 columns, 156 VGPRs and
-    // 3 waves with 512 lanes
-    if (tl == 2) {
-      if constexpr (F32) return launch_tb<T, C, 5, 896, 64, 32, 2, true>(a, st);
-      else return launch_tb<T, C, 5, 640, 64, 16, 2, true>(a, st);
-    }
-    // depth 4, coefficient hand-off on 1024 lanes (512^3, 256-plane chunks, one box):
-    //   bf16 coefficients, 64 x 32 tile (3 columns per lane, 117 VGPRs): 388 GLUP/s,
-    //   against 274 re-reading them on 512 lanes;
-    //   FP32 coefficients, 64 x 16 tile (2 columns, 110 VGPRs): 284 against 206 (896
-    //   lanes re-reading them) and 221 at depth 2; a 64 x 32 tile spills;
-    //   FP64, 64 x 8 tile (1 column, 110 VGPRs): 128 against 79 re-reading them on 512
-    //   lanes and 104 at depth 2; 896 lanes (2 columns) spill.
-    if (tl == 4) {
-      if constexpr (B16) return launch_tb<T, C, 5, 1024, 64, 32, 4, true>(a, st);
-      else if constexpr (F32) return launch_tb<T, C, 5, 1024, 64, 16, 4, true>(a, st);
-      else return launch_tb<T, C, 5, 1024, 64, 8, 4, true>(a, st);
-    }
-    // depth 6: bf16 with the hand-off, 1024 lanes, 64 x 16 (110 VGPRs): 322 against 227;
-    // the FP32 hand-off spills at this depth
-    if (tl == 6) {
-      if constexpr (B16) return launch_tb<T, C, 5, 1024, 64, 16, 6, true>(a, st);
-      else return launch_tb<T, C, 5, 512, 64, 16, 6>(a, st);
-    }
-  }
-  return hipErrorInvalidValue;
-}
-
-template <typename T, typename C>
-static hipError_t tb_pass_t(const Problem &P, int tl, const void *Y, void *ZN, const void *src, long long src_idx,
-                            const LaunchCfg &lc, hipStream_t st) {
+template <typename T>
+static hipError_t tb6_pass(const Problem &P, const void *Y, void *ZN, const void *src, long long src_idx,
+                           const LaunchCfg &lc, hipStream_t st) {
   const long long sz = (long long)P.pitch * P.rows;
-  TbArgs<T, C> a{};
+  TbArgs<T> a{};
   a.Y = (const T *)Y;
   a.ZN = (T *)ZN;
-  a.coef = (const C *)P.coef;
+  a.coef = (const T *)P.coef;
   a.cstride = P.field_elems;
   a.sy = P.pitch;
   a.sz = sz;
@@ -384,10 +300,12 @@ static hipError_t tb_pass_t(const Problem &P, int tl, const void *Y, void *ZN, c
   a.src = (const T *)src;
   a.src_k = src_idx < 0 ? -1 : (int)(src_idx / sz);
   a.src_off = src_idx < 0 ? 0 : (int)(src_idx % sz);
-  return tb_dispatch<T, C>(P.kernel, tl, a, st);
+  return launch_tb<T, 5, 512, 64, 16, 6>(a, st);
 }
 
 thread_local int *g_fused_tile_probe = nullptr;
+
+int fused_tiles(const Problem &P, int tl) { return P.kernel == 5 ? k5_tiles(P, tl) : 1; }
 
 bool fused_tile(const Problem &P, int tl, const LaunchCfg &lc, int *tx, int *ty) {
   int t[2] = {0, 0};
@@ -409,9 +327,12 @@ hipError_t tblock_pass(const Problem &P, int tl, const void *X, const void *Y, v
     return wave2_pass(P, X, Y, ZO, ZN, src, src_idx, lc, st);
   }
   if (P.kernel == 1) return jacobi_tb_pass(P, tl, Y, ZN, src, src_idx, lc, st);
-  if (P.dtype == GR_F64) return tb_pass_t<double, double>(P, tl, Y, ZN, src, src_idx, lc, st);
-  if (P.flags & GR_COEF_BF16) return tb_pass_t<float, __hip_bfloat16>(P, tl, Y, ZN, src, src_idx, lc, st);
-  return tb_pass_t<float, float>(P, tl, Y, ZN, src, src_idx, lc, st);
+  if (P.kernel != 5) return hipErrorInvalidValue;
+  if (tl == 6 && !(P.flags & GR_COEF_BF16)) {
+    if (P.dtype == GR_F64) return tb6_pass<double>(P, Y, ZN, src, src_idx, lc, st);
+    return tb6_pass<float>(P, Y, ZN, src, src_idx, lc, st);
+  }
+  return k5_pass(P, tl, Y, ZN, src, src_idx, lc, st);
 }
 
 }  // namespace gr

@@ -149,7 +149,8 @@ int gr_init_coef_uniform(gr_handle *h, uint64_t seed, double lo0, double hi0, do
                          double hi1);
 
 /* Launch configuration: tile variant of the sweep kernel (0 = default; see
- * gr_get_stats for the resulting tile), z planes streamed per workgroup (0 = all),
+ * gr_get_stats for the resulting tile; where a fused depth has several output tiles,
+ * variants 1, 2, .. below their number select those too), z planes streamed per workgroup (0 = all),
  * fused time steps per HBM pass (1 = single sweep; kernel 0: 2; kernel 1: 2..6;
  * kernel 5: 2, 4, 6; other depths return GR_EUNSUPPORTED).  Fused passes run only
  * while U1 and U2 hold the same halo (with GR_COEF_BF16: kernels 0 and 5);
