@@ -842,11 +842,32 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
         best_lc = top[i];
       }
   }
+  const float sweep_ms = best_ms;
   // stage 3: fused passes (time per application) on the scratch copies; kernel 0
   // reads the fields themselves (never written here) and writes the scratch pair
   {
     int depths[8];
     const int nd = tb_depths(P.kernel, P.dtype, depths, 8);
+    std::vector<std::pair<float, LaunchCfg>> fused;
+    // one untimed pass, then npass timed passes: ms per `steps` applications, comparable with the sweep trials
+    auto time_passes = [&](const LaunchCfg &lc, int npass, float *per_step) -> int {
+      const int tl = lc.t_block;
+      auto pass = [&](int q) {
+        if (P.kernel == 0) return tblock_pass(P, tl, ubase(h, 0), ubase(h, 1), a, b, nullptr, -1, lc, h->stream);
+        return tblock_pass(P, tl, nullptr, q & 1 ? b : a, nullptr, q & 1 ? a : b, nullptr, -1, lc, h->stream);
+      };
+      hipError_t e = pass(0);
+      if (e != hipSuccess) return fail(GR_EHIP, "autotune fused launch: %s", hipGetErrorString(e));
+      HIP_TRY(hipEventRecord(h->ev0, h->stream));
+      for (int q = 1; q <= npass; ++q)
+        if ((e = pass(q)) != hipSuccess) return fail(GR_EHIP, "autotune fused launch: %s", hipGetErrorString(e));
+      HIP_TRY(hipEventRecord(h->ev1, h->stream));
+      HIP_TRY(hipEventSynchronize(h->ev1));
+      float ms = 0.f;
+      HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
+      *per_step = ms * steps / (float)(npass * tl);
+      return GR_OK;
+    };
     for (int i = 0; i < nd; ++i) {
       bool ok = false;
       if ((rc = fused_depth_ok(h, depths[i], &ok))) return rc;
@@ -854,54 +875,65 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
       const int tl = depths[i];
       const int npass = (steps + tl - 1) / tl;
       for (int ft = 0; ft < fused_tiles(P, tl); ++ft) {
-      std::vector<int> zcs;
-      {  // first the chunks that make the workgroups one to four full rounds of the GPU's CUs
         LaunchCfg lc = best_lc;
+        lc.t_block = tl;
         lc.ftile = ft;
+        // chunk lengths: first those that make the workgroups one to four full rounds of
+        // the GPU's CUs (at 512^3 they are up to 15% faster than the powers of two)
+        std::vector<int> zcs;
+        auto add = [&](int zc) {
+          if (std::find(zcs.begin(), zcs.end(), zc) == zcs.end()) zcs.push_back(zc);
+        };
         int tx = 0, ty = 0;
         if (fused_tile(P, tl, lc, &tx, &ty)) {
           const int ntile = ((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty);
           for (int r = 1; r <= 4; ++r) {
-            const int nzc = r * ncu / ntile;
-            const int zc = nzc > 0 ? (nz + nzc - 1) / nzc : 0;
-            if (zc >= 2 * tl && zc < nz && std::find(zcs.begin(), zcs.end(), zc) == zcs.end()) zcs.push_back(zc);
+            const int nzc = r * ncu / ntile, zc = nzc > 0 ? (nz + nzc - 1) / nzc : 0;
+            if (zc >= 2 * tl && zc < nz) add(zc);
           }
         }
-        for (int zc : zchunks)
-          if (std::find(zcs.begin(), zcs.end(), zc) == zcs.end()) zcs.push_back(zc);
-      }
-      // (a tile whose first chunk lengths are far from the best so far skips the others)
-      float tile_ms = 1e30f;
-      for (size_t iz = 0; iz < zcs.size() && !(iz >= 2 && tile_ms > 1.4f * best_ms); ++iz)
-      for (int order = 0; order < 3; ++order) {  // XCD-contiguous orders keep the margins' re-reads in one L2
-        const int zc = zcs[iz];
-        LaunchCfg lc = best_lc;
-        lc.ftile = ft;
-        lc.t_block = tl;
-        lc.zchunk = zc;
-        lc.xcd_order = order;
-        auto pass = [&]() {
-          if (P.kernel == 0) return tblock_pass(P, tl, ubase(h, 0), ubase(h, 1), a, b, nullptr, -1, lc, h->stream);
-          return tblock_pass(P, tl, nullptr, b, nullptr, a, nullptr, -1, lc, h->stream);
-        };
-        hipError_t e = pass();
-        if (e != hipSuccess) return fail(GR_EHIP, "autotune fused launch: %s", hipGetErrorString(e));
-        HIP_TRY(hipEventRecord(h->ev0, h->stream));
-        for (int q = 0; q < npass; ++q)
-          if ((e = pass()) != hipSuccess) return fail(GR_EHIP, "autotune fused launch: %s", hipGetErrorString(e));
-        HIP_TRY(hipEventRecord(h->ev1, h->stream));
-        HIP_TRY(hipEventSynchronize(h->ev1));
-        float ms = 0.f;
-        HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
-        const float per_step = ms * steps / (float)(npass * tl);  // comparable with the sweep trials
-        tile_ms = std::min(tile_ms, per_step);
-        if (per_step < best_ms) {
-          best_ms = per_step;
-          best_lc = lc;
-        }
-      }
+        for (int zc : zchunks) add(zc);
+        // two lengths in every order (XCD-contiguous orders keep the margins' re-reads in
+        // one L2), then the others in the tile's best order, unless the tile is far from
+        // the best configuration so far
+        float tile_ms = 1e30f;
+        int tile_order = 0;
+        for (size_t iz = 0; iz < zcs.size() && !(iz >= 2 && tile_ms > 1.4f * best_ms); ++iz)
+          for (int order = 0; order < 3; ++order) {
+            if (iz >= 2 && order != tile_order) continue;
+            lc.zchunk = zcs[iz];
+            lc.xcd_order = order;
+            float ms = 0.f;
+            if ((rc = time_passes(lc, npass, &ms))) return rc;
+            fused.emplace_back(ms, lc);
+            if (ms < tile_ms) {
+              tile_ms = ms;
+              tile_order = order;
+            }
+            best_ms = std::min(best_ms, ms);
+          }
       }
     }
+    // the four fastest again, over four times as many applications, as in stage 2b
+    std::stable_sort(fused.begin(), fused.end(),
+                     [](const std::pair<float, LaunchCfg> &x, const std::pair<float, LaunchCfg> &y) {
+                       return x.first < y.first;
+                     });
+    const size_t ntop = std::min<size_t>(4, fused.size());
+    float tmin[4] = {1e30f, 1e30f, 1e30f, 1e30f};
+    for (int round = 0; round < 2; ++round)
+      for (size_t i = 0; i < ntop; ++i) {
+        if (fused[i].first > 1.1f * best_ms) continue;
+        float ms = 0.f;
+        if ((rc = time_passes(fused[i].second, std::max(3, 4 * steps / fused[i].second.t_block), &ms))) return rc;
+        tmin[i] = std::min(tmin[i], ms);
+      }
+    best_ms = sweep_ms;
+    for (size_t i = 0; i < ntop; ++i)
+      if (tmin[i] < best_ms) {
+        best_ms = tmin[i];
+        best_lc = fused[i].second;
+      }
   }
   h->spares_synced = true;  // the scratch pair holds tuning garbage in the interior; halos still match
   h->lc = best_lc;

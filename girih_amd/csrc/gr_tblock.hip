@@ -26,8 +26,8 @@
 // six planes of coefficients do not fit the registers and every level reads its own
 // again: level t = f(level t-1), input Y, output ZN.  The other depths of kernel 5 keep
 // them on chip (gr_star7.hpp; at depth 6 that form, reading them at every level, ran 121
-// against 183-198 GLUP/s here in FP32 at 512^3).  Kernel 1 has a leaner pass in
-// gr_fused1.hip and kernel 0 (second order in time) a two-step pass in gr_wave2.hip.
+// against 183-198 GLUP/s here in FP32 at 512^3), kernel 1 runs there too, and kernel 0
+// (second order in time) has a two-step pass in gr_wave2.hip.
 #include <hip/hip_runtime.h>
 
 #include "../../include/girih_gpu.h"
@@ -269,7 +269,7 @@ int tb_depths(int kid, int dtype, int *out, int max) {
     if (n < max) out[n++] = d;
   };
   (void)dtype;
-  if (kid == 1) {  // gr_fused1.hip
+  if (kid == 1) {  // gr_star7_k1_f32.hip, gr_star7_k1_f64.hip
     for (int d = 2; d <= 6; ++d) add(d);
   } else if (kid == 5) {  // gr_star7_k5.hip; depth 6 without bf16 coefficients: tb_kernel
     add(2);
@@ -305,7 +305,14 @@ static hipError_t tb6_pass(const Problem &P, const void *Y, void *ZN, const void
 
 thread_local int *g_fused_tile_probe = nullptr;
 
-int fused_tiles(const Problem &P, int tl) { return P.kernel == 5 ? k5_tiles(P, tl) : 1; }
+int fused_tiles(const Problem &P, int tl) {
+  if (P.kernel == 5) return k5_tiles(P, tl);
+  if (P.kernel == 1) {
+    if (P.dtype == GR_F64) return tl == 2 || tl == 4 ? 2 : 1;
+    return tl == 2 || tl == 3 ? 2 : tl == 4 ? 3 : 1;
+  }
+  return 1;
+}
 
 bool fused_tile(const Problem &P, int tl, const LaunchCfg &lc, int *tx, int *ty) {
   int t[2] = {0, 0};
@@ -326,7 +333,9 @@ hipError_t tblock_pass(const Problem &P, int tl, const void *X, const void *Y, v
     if (tl != 2) return hipErrorInvalidValue;
     return wave2_pass(P, X, Y, ZO, ZN, src, src_idx, lc, st);
   }
-  if (P.kernel == 1) return jacobi_tb_pass(P, tl, Y, ZN, src, src_idx, lc, st);
+  if (P.kernel == 1)
+    return P.dtype == GR_F64 ? k1_pass_f64(P, tl, Y, ZN, src, src_idx, lc, st)
+                             : k1_pass_f32(P, tl, Y, ZN, src, src_idx, lc, st);
   if (P.kernel != 5) return hipErrorInvalidValue;
   if (tl == 6 && !(P.flags & GR_COEF_BF16)) {
     if (P.dtype == GR_F64) return tb6_pass<double>(P, Y, ZN, src, src_idx, lc, st);

@@ -13,7 +13,9 @@ from test_gpu_parity import _bf16_round, _consts, _pad, _pad_coef, _random_probl
 pytestmark = pytest.mark.gpu
 
 # (kernel, storage, depth, tile variants of that depth)
-PASSES = [(5, "f64", 2, 1), (5, "f64", 4, 1), (5, "f32", 2, 2), (5, "f32", 4, 1), (5, "bf16", 2, 1), (5, "bf16", 4, 3),
+PASSES = [(1, "f32", 2, 2), (1, "f32", 3, 2), (1, "f32", 4, 3), (1, "f32", 5, 1), (1, "f32", 6, 1), (1, "f64", 2, 2),
+          (1, "f64", 3, 1), (1, "f64", 4, 2), (1, "f64", 5, 1), (1, "f64", 6, 1),
+          (5, "f64", 2, 1), (5, "f64", 4, 1), (5, "f32", 2, 2), (5, "f32", 4, 1), (5, "bf16", 2, 1), (5, "bf16", 4, 3),
           (5, "bf16", 6, 1), (5, "f32", 6, 1), (5, "f64", 6, 1)]
 # nx = 31, 63: the last halo cell is the last word of its row's pitch; 129 and 65 cross a tile by one cell
 GRIDS = [(31, 9, 5), (63, 17, 9), (129, 33, 7), (66, 65, 3), (3, 2, 1)]
@@ -37,6 +39,7 @@ def test_pass_edges_bitexact(kernel, storage, depth, tiles, zchunk, order):
                 st.upload(_pad(u), _pad(v), None, _pad_coef(coef, kernel))
                 if n > 0:
                     st.set_source(*pt, src)
+                st.set_streaming(n % 2)  # both cache policies of the kernel-1 passes
                 st.set_config(tile, zchunk, depth)
                 st.set_xcd_order(order)
                 st.step(napply)
