@@ -53,14 +53,14 @@ int fused_tiles(const Problem &P, int tl);
 hipError_t tblock_pass(const Problem &P, int tl, const void *X, const void *Y, void *ZO, void *ZN, const void *src,
                        long long src_idx, const LaunchCfg &lc, hipStream_t st);
 int tb_depths(int kid, int dtype, int *out, int max);
-// tl kernel-5 steps per pass (Y -> Z), and the output tiles of that depth.
-hipError_t k5_pass(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+// tl kernel-5 steps per pass (Y -> Z; level tl-1 -> Z1 unless null), and the output tiles of that depth.
+hipError_t k5_pass(const Problem &P, int tl, const void *Y, void *Z1, void *Z, const void *src, long long src_idx,
                    const LaunchCfg &lc, hipStream_t st);
 int k5_tiles(const Problem &P, int tl);
-// tl kernel-1 steps per pass: Y -> Z.
-hipError_t k1_pass_f32(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+// tl kernel-1 steps per pass: Y -> Z (level tl-1 -> Z1 unless null).
+hipError_t k1_pass_f32(const Problem &P, int tl, const void *Y, void *Z1, void *Z, const void *src, long long src_idx,
                        const LaunchCfg &lc, hipStream_t st);
-hipError_t k1_pass_f64(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+hipError_t k1_pass_f64(const Problem &P, int tl, const void *Y, void *Z1, void *Z, const void *src, long long src_idx,
                        const LaunchCfg &lc, hipStream_t st);
 // Two kernel-0 steps per pass: (X, Y) = (u^(n-1), u^n) -> (ZO, ZN) = (u^(n+1), u^(n+2)).
 hipError_t wave2_pass(const Problem &P, const void *X, const void *Y, void *ZO, void *ZN, const void *src,

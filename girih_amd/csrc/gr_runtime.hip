@@ -196,6 +196,7 @@ struct gr_handle {
   long long napplied = 0;
   gr_stats stats{};
   int device = 0;
+  int ncu = 1;         // compute units of the device
   // graph mode (gr_set_graph): the last captured step sequence and the state it leaves
   bool use_graph = false;
   hipGraphExec_t gexec = nullptr;
@@ -290,7 +291,9 @@ extern "C" int gr_create(const gr_desc *d, gr_handle **out) {
   const size_t fbytes = (size_t)P.field_elems * es;
   hipError_t e;
   int rc = GR_OK;
-  if ((e = hipGetDevice(&h->device)) != hipSuccess) rc = fail(GR_EHIP, "hipGetDevice: %s", hipGetErrorString(e));
+  if ((e = hipGetDevice(&h->device)) != hipSuccess ||
+      (e = hipDeviceGetAttribute(&h->ncu, hipDeviceAttributeMultiprocessorCount, h->device)) != hipSuccess)
+    rc = fail(GR_EHIP, "hipGetDevice: %s", hipGetErrorString(e));
   // Zero fills go on the handle's own (non-blocking) stream, which does not order with
   // the null stream: a null-stream hipMemset could still be running when the first
   // kernel on the handle's stream writes the same memory.
@@ -467,7 +470,8 @@ extern "C" int gr_set_source(gr_handle *h, int i, int j, int k, const double *va
 }
 
 static int check_halo_equal(gr_handle *h);
-static int ensure_spares(gr_handle *h);
+static int ensure_spares(gr_handle *h, int n = 2);
+static int sync_spares(gr_handle *h);
 static int enqueue_apps(gr_handle *h, int napply, bool fuse, int *nlaunch);
 static int finish_step(gr_handle *h, int napply, int launches);
 static void drop_graph(gr_handle *h) {
@@ -510,22 +514,20 @@ static int fused_depth_ok(gr_handle *h, int tl, bool *ok) {
 extern "C" int gr_step(gr_handle *h, int napply) {
   if (!h) return fail(GR_EINVAL, "gr_step: null handle");
   if (napply < 0) return fail(GR_EINVAL, "gr_step: negative step count");
-  const Problem &P = h->P;
-  const size_t es = elem_size(P.dtype);
   const int tl = h->lc.t_block;
   bool fuse = false;
   int rc = fused_depth_ok(h, tl, &fuse);
   if (rc) return rc;
-  const bool wave = P.kernel == 0;
+  const bool wave = h->P.kernel == 0;
   if (fuse && wave) {
-    if ((rc = ensure_spares(h))) return rc;
-    if (!h->spares_synced) {  // spares need the fields' halo (never written by a pass)
-      int sp[2];
-      spare_ids(h, sp);
-      const size_t fbytes = (size_t)P.field_elems * es;
-      HIP_TRY(hipMemcpyAsync(h->fbuf[sp[0]], h->fbuf[h->lu[1]], fbytes, hipMemcpyDeviceToDevice, h->stream));
-      HIP_TRY(hipMemcpyAsync(h->fbuf[sp[1]], h->fbuf[h->lu[1]], fbytes, hipMemcpyDeviceToDevice, h->stream));
-      h->spares_synced = true;
+    if ((rc = ensure_spares(h)) || (rc = sync_spares(h))) return rc;
+  } else if (fuse) {
+    // a third buffer lets the last pass write both levels that a call leaves; without the
+    // memory for it a call ends with a single sweep
+    if (ensure_spares(h, 1) == GR_OK) {
+      if ((rc = sync_spares(h))) return rc;
+    } else {
+      (void)hipGetLastError();
     }
   }
   // graph mode: replay the launch sequence of an identical earlier call
@@ -573,6 +575,89 @@ extern "C" int gr_step(gr_handle *h, int napply) {
   return finish_step(h, napply, launches);
 }
 
+// The z chunk with which a pass of depth tl has at most `rounds` workgroups per CU, as
+// near to that as whole chunks allow (0: the whole z, or chunks shorter than 2*tl planes,
+// which would mostly compute each other's ghost planes).
+static int round_chunk(const gr_handle *h, int tl, const LaunchCfg &lc, int rounds) {
+  const Problem &P = h->P;
+  int tx = 0, ty = 0;
+  if (!fused_tile(P, tl, lc, &tx, &ty)) return 0;
+  const int ntile = ((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty);
+  const int nzc = rounds * h->ncu / ntile, zc = nzc > 0 ? (P.nz + nzc - 1) / nzc : 0;
+  return zc >= 2 * tl && zc < P.nz ? zc : 0;
+}
+
+// Launch napply applications of a first-order kernel as fused passes, the last of which
+// writes the field's last two levels (the U1/U2 pair a call leaves) into different
+// buffers, so that no single sweep is needed to make both exact: at 512^3, 20 kernel-5
+// FP64 steps at depth 4 were 4 passes and 4 sweeps, and the sweeps took 40% of the time.
+// A rest shorter than the depth runs as one shallower pass, and as a sweep where one
+// application is left.  Three buffers take part: U1, U2 and a spare.  A pass may write
+// any buffer but the one it reads, so the sequence is led such that the call ends on
+// the buffers it began with (a captured graph then stays valid); only a call of one
+// pass has to trade the read field for the spare.
+static int enqueue_first_order(gr_handle *h, int napply, int *nlaunch) {
+  const Problem &P = h->P;
+  const size_t es = elem_size(P.dtype);
+  int depths[8];
+  const int nd = tb_depths(P.kernel, P.dtype, depths, 8);
+  std::vector<int> ops;  // depth of each launch (1: a single sweep)
+  for (int rest = napply; rest > 0; rest -= ops.back()) {
+    int d = 1;
+    for (int i = 0; i < nd; ++i)
+      if (depths[i] <= std::min(rest, h->lc.t_block)) d = std::max(d, depths[i]);
+    ops.push_back(d);
+  }
+  int sp[2];
+  spare_ids(h, sp);
+  const int m = (int)ops.size(), w = h->parity, r = 1 - w;
+  const int newest = (napply & 1) ? w : r;            // the logical field that ends newest
+  int end[2] = {h->lu[0], h->lu[1]};                   // buffers of U1 and U2 after the call
+  const bool both = m > 0 && ops[m - 1] > 1;           // the last launch writes both levels
+  int x = h->lu[r];                                    // buffer read next
+  if (m == 1 && both) end[r] = sp[0];                  // one pass reads end[r]'s buffer
+  if (m == 2 && !both && newest == w) end[r] = sp[0];  // one pass and one sweep: the same
+  // the buffer the last launch reads: for a pass the one that stays free, for a sweep the older level's
+  const int last_in = both ? (m == 1 ? x : sp[0]) : end[1 - newest];
+  long long app = h->napplied;
+  for (int i = 0; i < m; ++i) {
+    const bool has_src = h->src && app < h->nsrc;
+    const void *srcp = has_src ? (const char *)h->src + (size_t)app * es : nullptr;
+    const long long sidx = has_src ? h->src_idx : -1;
+    LaunchCfg lc = h->lc;
+    if (ops[i] != lc.t_block) {  // a shallower pass: its own tile, and chunks for one round of the CUs
+      lc.ftile = 0;
+      if (ops[i] > 1) lc.zchunk = round_chunk(h, ops[i], lc, 1);
+    }
+    const void *in = field_base(h, h->fbuf[x]);
+    hipError_t e;
+    if (i == m - 1) {
+      void *out = field_base(h, h->fbuf[end[newest]]);
+      e = both ? tblock_pass(P, ops[i], nullptr, in, field_base(h, h->fbuf[end[1 - newest]]), out, srcp, sidx, lc,
+                             h->stream)
+               : sweep_fields(P, out, in, srcp, sidx, lc, h->stream);
+    } else {
+      // the next buffer: any other one, such that the last launch finds its input in last_in
+      int y = last_in;
+      if (i < m - 2 || y == x)
+        for (int c : {h->lu[w], h->lu[r], sp[0]})
+          if (c != x && (i < m - 3 || c != last_in)) {
+            y = c;
+            break;
+          }
+      e = tblock_pass(P, ops[i], nullptr, in, nullptr, field_base(h, h->fbuf[y]), srcp, sidx, lc, h->stream);
+      x = y;
+    }
+    if (e != hipSuccess) return fail(GR_EHIP, "fused pass launch failed: %s", hipGetErrorString(e));
+    app += ops[i];
+  }
+  h->parity ^= napply & 1;
+  h->lu[0] = end[0];
+  h->lu[1] = end[1];
+  *nlaunch = m;
+  return GR_OK;
+}
+
 // Launch napply applications on the handle's stream (fused passes where enabled,
 // then single sweeps), advancing the host-side parity and buffer mapping.  Only
 // kernel launches: the sequence may be captured into a HIP graph.
@@ -582,6 +667,11 @@ static int enqueue_apps(gr_handle *h, int napply, bool fuse, int *nlaunch) {
   const int tl = h->lc.t_block;
   const bool wave = P.kernel == 0;
   int s = 0, launches = 0;
+  if (fuse && !wave && napply > 1) {
+    int sp[2];
+    spare_ids(h, sp);
+    if (h->fbuf[sp[0]]) return enqueue_first_order(h, napply, nlaunch);
+  }
   if (fuse) {
     // kernel 0 keeps (u^(n-1), u^n) exact after every pass; first-order kernels
     // keep the last application as a single sweep so U1 and U2 end exact.
@@ -724,9 +814,10 @@ extern "C" int gr_set_xcd_order(gr_handle *h, int xcd_order) {
   return GR_OK;
 }
 
-static int ensure_spares(gr_handle *h) {
+// The first n spare buffers.
+static int ensure_spares(gr_handle *h, int n) {
   const size_t fbytes = (size_t)h->P.field_elems * elem_size(h->P.dtype);
-  for (int i = 2; i < 4; ++i)
+  for (int i = 2; i < 2 + n; ++i)
     if (!h->fbuf[i]) {
       drop_graph(h);
       HIP_TRY(hipMalloc(&h->fbuf[i], fbytes));
@@ -751,8 +842,6 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
   h->spares_synced = true;  // copies of the fields: same halo
   void *a = field_base(h, h->fbuf[sp[0]]), *b = field_base(h, h->fbuf[sp[1]]);
   const int nz = P.nz;
-  int ncu = 0;
-  HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device));
   std::vector<int> zchunks = {0};
   for (int zc : {512, 256, 128, 64, 32})
     if (zc < nz) zchunks.push_back(zc);
@@ -884,13 +973,9 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
         auto add = [&](int zc) {
           if (std::find(zcs.begin(), zcs.end(), zc) == zcs.end()) zcs.push_back(zc);
         };
-        int tx = 0, ty = 0;
-        if (fused_tile(P, tl, lc, &tx, &ty)) {
-          const int ntile = ((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty);
-          for (int r = 1; r <= 4; ++r) {
-            const int nzc = r * ncu / ntile, zc = nzc > 0 ? (nz + nzc - 1) / nzc : 0;
-            if (zc >= 2 * tl && zc < nz) add(zc);
-          }
+        for (int r = 1; r <= 4; ++r) {
+          const int zc = round_chunk(h, tl, lc, r);
+          if (zc > 0) add(zc);
         }
         for (int zc : zchunks) add(zc);
         // two lengths in every order (XCD-contiguous orders keep the margins' re-reads in
@@ -1072,20 +1157,37 @@ __global__ void init_fields_kernel(T *u1, T *u2, T *r2, int mode, uint64_t seed,
   u2[o] = val;
 }
 
+// f(offset) for every halo cell (outside the interior box) of a field, one wavefront per
+// row: all cells of a row in the y or z halo, else the R cells at both ends.
+template <typename F>
+__device__ __forceinline__ void for_halo_cells(int nx, int ny, int nz, int R, long long pitch, F &&f) {
+  const long long rows = ny + 2 * R, row = (long long)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
+  const int lane = threadIdx.x % 64, j = (int)(row % rows), k = (int)(row / rows);
+  if (k >= nz + 2 * R) return;
+  const long long o = row * pitch;
+  if (j >= R && j < ny + R && k >= R && k < nz + R) {
+    if (lane < 2 * R) f(o + (lane < R ? lane : nx + lane));
+  } else {
+    for (int i = lane; i < nx + 2 * R; i += 64) f(o + i);
+  }
+}
+
 // flag = 1 if U1 and U2 differ (bitwise) anywhere outside the interior box
 template <typename U>
-__global__ void halo_diff_kernel(const U *a, const U *b, int nx, int ny, int nz, int R, long long pitch, long long rows,
-                                 long long total, int *flag) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= total) return;
-  const int nnx = nx + 2 * R;
-  const long long row = t / nnx;
-  const int i = (int)(t - row * nnx);
-  const int j = (int)(row % rows);
-  const int k = (int)(row / rows);
-  const bool inner = i >= R && i < nx + R && j >= R && j < ny + R && k >= R && k < nz + R;
-  const long long o = row * pitch + i;
-  if (!inner && a[o] != b[o]) *flag = 1;
+__global__ void halo_diff_kernel(const U *a, const U *b, int nx, int ny, int nz, int R, long long pitch, int *flag) {
+  for_halo_cells(nx, ny, nz, R, pitch, [&](long long o) {
+    if (a[o] != b[o]) *flag = 1;
+  });
+}
+
+// the halo of src into d0 (and d1 unless null)
+template <typename U>
+__global__ void halo_copy_kernel(const U *src, U *d0, U *d1, int nx, int ny, int nz, int R, long long pitch) {
+  for_halo_cells(nx, ny, nz, R, pitch, [&](long long o) {
+    const U v = src[o];
+    d0[o] = v;
+    if (d1) d1[o] = v;
+  });
 }
 
 // Coefficient m of halo-inclusive cell (i, j, k) is drawn from its logical index
@@ -1114,22 +1216,39 @@ static int check_halo_equal(gr_handle *h) {
   const Problem &P = h->P;
   if (!h->flag) HIP_TRY(hipMalloc(&h->flag, sizeof(int)));
   HIP_TRY(hipMemsetAsync(h->flag, 0, sizeof(int), h->stream));
-  const long long total = (long long)(P.nx + 2 * P.R) * P.rows * P.planes;
   const int bs = 256;
-  const unsigned nb = (unsigned)((total + bs - 1) / bs);
+  const unsigned nb = (unsigned)(((long long)P.rows * P.planes + 3) / 4);
   if (P.dtype == GR_F64)
     hipLaunchKernelGGL(halo_diff_kernel<unsigned long long>, dim3(nb), dim3(bs), 0, h->stream,
                        (const unsigned long long *)ubase(h, 0), (const unsigned long long *)ubase(h, 1), P.nx, P.ny,
-                       P.nz, P.R, (long long)P.pitch, (long long)P.rows, total, (int *)h->flag);
+                       P.nz, P.R, (long long)P.pitch, (int *)h->flag);
   else
     hipLaunchKernelGGL(halo_diff_kernel<unsigned>, dim3(nb), dim3(bs), 0, h->stream, (const unsigned *)ubase(h, 0),
-                       (const unsigned *)ubase(h, 1), P.nx, P.ny, P.nz, P.R, (long long)P.pitch, (long long)P.rows,
-                       total, (int *)h->flag);
+                       (const unsigned *)ubase(h, 1), P.nx, P.ny, P.nz, P.R, (long long)P.pitch, (int *)h->flag);
   HIP_TRY(hipGetLastError());
   int hflag = 1;
   HIP_TRY(hipMemcpyAsync(&hflag, h->flag, sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
   h->halo_equal = hflag == 0 ? 1 : 0;
+  return GR_OK;
+}
+
+// The spares get the fields' halo, which passes read but never write.
+static int sync_spares(gr_handle *h) {
+  if (h->spares_synced) return GR_OK;
+  const Problem &P = h->P;
+  int sp[2];
+  spare_ids(h, sp);
+  const unsigned nb = (unsigned)(((long long)P.rows * P.planes + 3) / 4);
+  void *d0 = field_base(h, h->fbuf[sp[0]]), *d1 = field_base(h, h->fbuf[sp[1]]);
+  if (P.dtype == GR_F64)
+    hipLaunchKernelGGL(halo_copy_kernel<double>, dim3(nb), dim3(256), 0, h->stream, (const double *)ubase(h, 1),
+                       (double *)d0, (double *)d1, P.nx, P.ny, P.nz, P.R, (long long)P.pitch);
+  else
+    hipLaunchKernelGGL(halo_copy_kernel<float>, dim3(nb), dim3(256), 0, h->stream, (const float *)ubase(h, 1),
+                       (float *)d0, (float *)d1, P.nx, P.ny, P.nz, P.R, (long long)P.pitch);
+  HIP_TRY(hipGetLastError());
+  h->spares_synced = true;
   return GR_OK;
 }
 
@@ -1391,14 +1510,9 @@ int gr_internal_fused_prepare(gr_handle *h, bool *ok) {
   int rc = fused_depth_ok(h, 2, &depth_ok);
   if (rc || !depth_ok || h->P.kernel != 0) return rc;
   if ((rc = ensure_spares(h))) return rc;
-  if (!h->spares_synced) {  // the spares need the fields' halo (never written by a pass)
-    int sp[2];
-    spare_ids(h, sp);
-    const size_t fbytes = (size_t)h->P.field_elems * elem_size(h->P.dtype);
-    HIP_TRY(hipMemcpyAsync(h->fbuf[sp[0]], h->fbuf[h->lu[1]], fbytes, hipMemcpyDeviceToDevice, h->stream));
-    HIP_TRY(hipMemcpyAsync(h->fbuf[sp[1]], h->fbuf[h->lu[1]], fbytes, hipMemcpyDeviceToDevice, h->stream));
+  if (!h->spares_synced) {
+    if ((rc = sync_spares(h))) return rc;
     HIP_TRY(hipStreamSynchronize(h->stream));
-    h->spares_synced = true;
   }
   *ok = true;
   return GR_OK;

@@ -34,9 +34,9 @@ static hipError_t k1_dispatch(int tl, int tile, const S7Args<float, float> &a, h
   }
 }
 
-hipError_t k1_pass_f32(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+hipError_t k1_pass_f32(const Problem &P, int tl, const void *Y, void *Z1, void *Z, const void *src, long long src_idx,
                        const LaunchCfg &lc, hipStream_t st) {
-  const S7Args<float, float> a = s7_args<float, float>(P, Y, Z, src, src_idx, lc);
+  const S7Args<float, float> a = s7_args<float, float>(P, Y, Z1, Z, src, src_idx, lc);
   return streaming_sweep(P) ? k1_dispatch<true>(tl, lc.ftile, a, st) : k1_dispatch<false>(tl, lc.ftile, a, st);
 }
 

@@ -27,9 +27,9 @@ static hipError_t k1_dispatch(int tl, int tile, const S7Args<double, double> &a,
   }
 }
 
-hipError_t k1_pass_f64(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+hipError_t k1_pass_f64(const Problem &P, int tl, const void *Y, void *Z1, void *Z, const void *src, long long src_idx,
                        const LaunchCfg &lc, hipStream_t st) {
-  const S7Args<double, double> a = s7_args<double, double>(P, Y, Z, src, src_idx, lc);
+  const S7Args<double, double> a = s7_args<double, double>(P, Y, Z1, Z, src, src_idx, lc);
   return streaming_sweep(P) ? k1_dispatch<true>(tl, lc.ftile, a, st) : k1_dispatch<false>(tl, lc.ftile, a, st);
 }
 

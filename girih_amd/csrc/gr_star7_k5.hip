@@ -54,20 +54,20 @@ int k5_tiles(const Problem &P, int tl) {
 }
 
 template <typename T, typename C>
-static hipError_t k5_pass_t(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+static hipError_t k5_pass_t(const Problem &P, int tl, const void *Y, void *Z1, void *Z, const void *src, long long src_idx,
                             const LaunchCfg &lc, hipStream_t st) {
-  S7Args<T, C> a = s7_args<T, C>(P, Y, Z, src, src_idx, lc);
+  S7Args<T, C> a = s7_args<T, C>(P, Y, Z1, Z, src, src_idx, lc);
   a.coef = (const C *)P.coef - P.xoff;  // addressed with the fields' element index
   a.cstride = P.field_elems;
   return k5_dispatch<T, C>(tl, lc.ftile, a, st);
 }
 
-// One pass of tl kernel-5 steps: Y -> Z.
-hipError_t k5_pass(const Problem &P, int tl, const void *Y, void *Z, const void *src, long long src_idx,
+// One pass of tl kernel-5 steps: Y -> Z (level tl-1 -> Z1 unless null).
+hipError_t k5_pass(const Problem &P, int tl, const void *Y, void *Z1, void *Z, const void *src, long long src_idx,
                    const LaunchCfg &lc, hipStream_t st) {
-  if (P.dtype == GR_F64) return k5_pass_t<double, double>(P, tl, Y, Z, src, src_idx, lc, st);
-  if (P.flags & GR_COEF_BF16) return k5_pass_t<float, __hip_bfloat16>(P, tl, Y, Z, src, src_idx, lc, st);
-  return k5_pass_t<float, float>(P, tl, Y, Z, src, src_idx, lc, st);
+  if (P.dtype == GR_F64) return k5_pass_t<double, double>(P, tl, Y, Z1, Z, src, src_idx, lc, st);
+  if (P.flags & GR_COEF_BF16) return k5_pass_t<float, __hip_bfloat16>(P, tl, Y, Z1, Z, src, src_idx, lc, st);
+  return k5_pass_t<float, float>(P, tl, Y, Z1, Z, src, src_idx, lc, st);
 }
 
 }  // namespace gr

@@ -16,20 +16,22 @@ static hipError_t launch_s7(S7Args<T, C> a, hipStream_t st) {
   a.zchunk = (a.zchunk <= 0 || a.zchunk > a.nz) ? a.nz : a.zchunk;
   a.nzc = (a.nz + a.zchunk - 1) / a.zchunk;
   const dim3 grid(a.tiles_x * a.tiles_y * a.nzc);
-  if (a.src_k >= 0)
+  if (a.src_k >= 0 || a.Z1)
     hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, STRM, true>), grid, dim3(NT), 0, st, a);
   else
     hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, STRM, false>), grid, dim3(NT), 0, st, a);
   return hipGetLastError();
 }
 
-// Arguments of a pass Y -> Z over problem P (fields given with the x offset applied).
+// Arguments of a pass Y -> Z over problem P (fields given with the x offset applied); Z1,
+// when given, receives level tl-1.
 template <typename T, typename C>
-static S7Args<T, C> s7_args(const Problem &P, const void *Y, void *Z, const void *src, long long src_idx,
+static S7Args<T, C> s7_args(const Problem &P, const void *Y, void *Z1, void *Z, const void *src, long long src_idx,
                             const LaunchCfg &lc) {
   S7Args<T, C> a{};
   a.Y = (const T *)Y - P.xoff;
   a.Z = (T *)Z - P.xoff;
+  a.Z1 = Z1 ? (T *)Z1 - P.xoff : nullptr;
   a.c0 = (T)P.c[0];
   a.c1 = (T)P.c[1];
   a.sz = (long long)P.pitch * P.rows;

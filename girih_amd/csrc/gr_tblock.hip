@@ -40,6 +40,7 @@ template <typename T>
 struct TbArgs {
   const T *Y;   // level 0
   T *ZN;        // level TL
+  T *ZO;        // level TL-1 (null: not written)
   const T *coef;
   long long cstride;
   long long sy, sz;
@@ -234,7 +235,12 @@ __global__ __launch_bounds__(NT) void tb_kernel(const TbArgs<T> a) {
           for (int j = 0; j < NCOL; ++j)
             if (colv[j]) Lt[lofs[j]] = qv[t < TL ? t : 0][j][sl];
         }
-        // output: level TL into ZN -- planes of the box
+        // output: level TL into ZN (and level TL-1 into ZO) -- planes of the box
+        if (t == TL - 1 && a.ZO && live && zin && p >= zs && p < ze) {
+#pragma unroll
+          for (int j = 0; j < NCOL; ++j)
+            if (outc[j]) stb<T>(a.ZO + (long long)p * a.sz, off[j], val[j]);
+        }
         if (t == TL && live && zin && p >= zs && p < ze) {
 #pragma unroll
           for (int j = 0; j < NCOL; ++j)
@@ -282,12 +288,13 @@ int tb_depths(int kid, int dtype, int *out, int max) {
 }
 
 template <typename T>
-static hipError_t tb6_pass(const Problem &P, const void *Y, void *ZN, const void *src, long long src_idx,
+static hipError_t tb6_pass(const Problem &P, const void *Y, void *ZO, void *ZN, const void *src, long long src_idx,
                            const LaunchCfg &lc, hipStream_t st) {
   const long long sz = (long long)P.pitch * P.rows;
   TbArgs<T> a{};
   a.Y = (const T *)Y;
   a.ZN = (T *)ZN;
+  a.ZO = (T *)ZO;
   a.coef = (const T *)P.coef;
   a.cstride = P.field_elems;
   a.sy = P.pitch;
@@ -325,7 +332,7 @@ bool fused_tile(const Problem &P, int tl, const LaunchCfg &lc, int *tx, int *ty)
   return true;
 }
 
-// One fused pass of tl levels.  Kernels 1 and 5: Y -> ZN (X, ZO unused).
+// One fused pass of tl levels.  Kernels 1 and 5: Y -> ZN, and level tl-1 -> ZO unless null (X unused).
 // Kernel 0 (tl = 2): (X, Y) = (u^(n-1), u^n) -> (ZO, ZN) = (u^(n+1), u^(n+2)).
 hipError_t tblock_pass(const Problem &P, int tl, const void *X, const void *Y, void *ZO, void *ZN, const void *src,
                        long long src_idx, const LaunchCfg &lc, hipStream_t st) {
@@ -334,14 +341,14 @@ hipError_t tblock_pass(const Problem &P, int tl, const void *X, const void *Y, v
     return wave2_pass(P, X, Y, ZO, ZN, src, src_idx, lc, st);
   }
   if (P.kernel == 1)
-    return P.dtype == GR_F64 ? k1_pass_f64(P, tl, Y, ZN, src, src_idx, lc, st)
-                             : k1_pass_f32(P, tl, Y, ZN, src, src_idx, lc, st);
+    return P.dtype == GR_F64 ? k1_pass_f64(P, tl, Y, ZO, ZN, src, src_idx, lc, st)
+                             : k1_pass_f32(P, tl, Y, ZO, ZN, src, src_idx, lc, st);
   if (P.kernel != 5) return hipErrorInvalidValue;
   if (tl == 6 && !(P.flags & GR_COEF_BF16)) {
-    if (P.dtype == GR_F64) return tb6_pass<double>(P, Y, ZN, src, src_idx, lc, st);
-    return tb6_pass<float>(P, Y, ZN, src, src_idx, lc, st);
+    if (P.dtype == GR_F64) return tb6_pass<double>(P, Y, ZO, ZN, src, src_idx, lc, st);
+    return tb6_pass<float>(P, Y, ZO, ZN, src, src_idx, lc, st);
   }
-  return k5_pass(P, tl, Y, ZN, src, src_idx, lc, st);
+  return k5_pass(P, tl, Y, ZO, ZN, src, src_idx, lc, st);
 }
 
 }  // namespace gr

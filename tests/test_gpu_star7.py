@@ -27,12 +27,13 @@ def test_pass_edges_bitexact(kernel, storage, depth, tiles, zchunk, order):
     dt = np.float64 if storage == "f64" else np.float32
     for tile in range(tiles):
         for n, (nx, ny, nz) in enumerate(GRIDS):
-            napply = 2 * depth + 1 + n % 3
-            print("star7", kernel, storage, depth, tile, (nx, ny, nz), zchunk, napply, flush=True)
+            # one pass; two; a rest of one, of two and (where there is such a depth) of three
+            calls = (depth, 2 * depth, depth + 1, 2 * depth + 2, depth, 3 * depth + 3)
+            print("star7", kernel, storage, depth, tile, (nx, ny, nz), zchunk, calls, flush=True)
             u, v, _, coef = _random_problem(kernel, nx, ny, nz, dt, 300 + n)
             if storage == "bf16":
                 coef = _bf16_round(coef)
-            src = np.linspace(0.5, -1.0, napply)
+            src = np.linspace(0.5, -1.0, 4 * depth + 3)  # ends inside a call
             pt = (nx, ny, nz) if n % 2 else (1 + nx // 2, 1, nz)  # the last interior cell, or on an edge
             with gpu.Stepper(kernel, nx, ny, nz, dtype=gpu.GR_F64 if storage == "f64" else gpu.GR_F32,
                              flags=gpu.GR_COEF_BF16 if storage == "bf16" else 0, coef=_consts(coef, kernel)) as st:
@@ -42,13 +43,16 @@ def test_pass_edges_bitexact(kernel, storage, depth, tiles, zchunk, order):
                 st.set_streaming(n % 2)  # both cache policies of the kernel-1 passes
                 st.set_config(tile, zchunk, depth)
                 st.set_xcd_order(order)
-                st.step(napply)
-                assert st.stats()["last_launches"] < napply
-                U1, U2 = st.download(_pad(u).shape)
-            for a in range(napply):
-                w, r = (u, v) if a % 2 == 0 else (v, u)
-                orc.sweep(kernel, coef, w, r, None)
-                if n > 0:
-                    w[pt[2], pt[1], pt[0]] += dt(src[a])
-            np.testing.assert_array_equal(U1[:, :, :u.shape[2]], u)
-            np.testing.assert_array_equal(U2[:, :, :u.shape[2]], v)
+                a = 0
+                for napply in calls:
+                    st.step(napply)
+                    assert st.stats()["last_launches"] < napply
+                    U1, U2 = st.download(_pad(u).shape)
+                    for a in range(a, a + napply):
+                        w, r = (u, v) if a % 2 == 0 else (v, u)
+                        orc.sweep(kernel, coef, w, r, None)
+                        if n > 0 and a < src.size:
+                            w[pt[2], pt[1], pt[0]] += dt(src[a])
+                    a += 1
+                    np.testing.assert_array_equal(U1[:, :, :u.shape[2]], u)
+                    np.testing.assert_array_equal(U2[:, :, :u.shape[2]], v)
