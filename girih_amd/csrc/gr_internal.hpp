@@ -27,9 +27,13 @@ struct LaunchCfg {
   int variant = 0;  // sweep tile variant (0 = default tile)
   int xcd_order = 1;  // renumber workgroups per XCD
   int ftile = 0;      // output tile of the fused pass, where its depth has several (fused_tiles)
+  // settings the caller has not made: sweeps go by sweep_cfg's rule, fused passes by gr_step's
+  bool auto_variant = false, auto_zchunk = false, auto_order = false;
 };
 
 int num_tile_variants(int kid, int dtype);
+// lc with its automatic settings replaced by those for a sweep of a box of nx x ny x nz cells.
+LaunchCfg sweep_cfg(int kid, const LaunchCfg &lc, int nx, int ny, int nz);
 void tile_of_variant(int kid, int dtype, int variant, int *tx, int *ty);
 
 size_t elem_size(int dtype);

@@ -96,9 +96,44 @@ void tile_of_variant(int kid, int dtype, int variant, int *tx, int *ty) {
   *ty = ok ? rows[variant] : 16;
 }
 
+// The settings of a sweep that nobody tuned (gr_sweep_dev, and steppers until gr_set_config,
+// gr_set_xcd_order or gr_autotune), by kernel and box.  Measured on the sweep entry
+// point over 32^3 .. 600 x 600 x 300 in FP32 and FP64 (times per call, with its synchronisation):
+//  * chunks: whole-z items leave most CUs idle (403 x 300 x 219 FP32: kernel 0 317 us against
+//    119, kernel 5 540 against 262).  Enough chunks for two 512-lane workgroups per CU
+//    (64^3 kernel 1 FP64: 54 us whole, 20 at 8 planes, 18 at 4), but not longer than the
+//    kernel gains from: 32 planes for kernel 0, whose chunks re-read 8 planes (512^3 FP32
+//    32 planes 486 us, 16 500), 16 for kernel 1 (512^3 FP32 247 us, 32 planes 248, 128
+//    251), 4 where coefficient arrays are streamed (600 x 600 x 300 kernel 5 FP64 4 planes
+//    1490 us, 8 1534, 16 1558; 403 x 300 x 219 kernel 4 384, 405, 419);
+//  * tile: 128 x 16 of 1024 lanes (for kernel 0 with the operand prefetch) where it overhangs
+//    the box no further than 64 x 16 does (256^3 kernel 0 FP32 60 us against 62, 512^3
+//    486 against 520; but 320^3 138 against 133) and there is work for 256 of them; else
+//    64 x 16 of 512 lanes (64^3 kernel 0 19 us against 22);
+//  * order: XCD bands of tile rows (403 x 300 x 219 kernel 3 157 us, plain runs 164).
+LaunchCfg sweep_cfg(int kid, const LaunchCfg &lc, int nx, int ny, int nz) {
+  LaunchCfg c = lc;
+  const bool hot = kid == 0 || kid == 1 || kid == 5;  // kernels with tile variants
+  if (lc.auto_variant) {
+    const bool wide = (nx + 127) / 128 * 2 == (nx + 63) / 64 && (long long)nx * ny * nz >= (1 << 21);
+    c.variant = !hot ? 0 : !wide ? 2 : kid == 0 ? 16 : 13;
+  }
+  if (lc.auto_zchunk) {
+    int tx = 64, ty = 16;
+    tile_of_variant(kid, 0, c.variant, &tx, &ty);
+    const long long tiles = (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
+    const int most = kid == 0 ? 32 : kid == 1 ? 16 : 4;
+    c.zchunk = (int)std::min<long long>(most, std::max<long long>(4, tiles * nz / (tx > 64 ? 256 : 512)));
+  }
+  if (lc.auto_order) c.xcd_order = 2;
+  c.auto_variant = c.auto_zchunk = c.auto_order = false;
+  return c;
+}
+
 // One sweep u <- f(v) with the handle's configuration.
 hipError_t sweep_fields(const Problem &P, void *u, const void *v, const void *src, long long src_idx,
-                        const LaunchCfg &lc, hipStream_t st, const void *uold) {
+                        const LaunchCfg &cfg, hipStream_t st, const void *uold) {
+  const LaunchCfg lc = sweep_cfg(P.kernel, cfg, P.nx, P.ny, P.nz);
   const bool fast = (P.flags & GR_FAST) != 0;
   const bool rocs = (P.flags & GR_ROC2_SCALAR) != 0;
   const bool bf16 = (P.flags & GR_COEF_BF16) != 0;
@@ -167,11 +202,11 @@ using namespace gr;
 
 // What a captured step sequence depends on besides the (fixed) field allocations.
 struct GraphKey {
-  int napply, parity, lu0, lu1, variant, zchunk, t_block, xcd_order, ftile, fuse;
+  int napply, parity, lu0, lu1, variant, zchunk, t_block, xcd_order, ftile, autos, fuse;
   long long napplied;  // -1 unless a source is active (its pointers are baked into the graph)
   bool operator==(const GraphKey &o) const {
     return napply == o.napply && parity == o.parity && lu0 == o.lu0 && lu1 == o.lu1 && variant == o.variant &&
-           zchunk == o.zchunk && t_block == o.t_block && xcd_order == o.xcd_order && ftile == o.ftile && fuse == o.fuse &&
+           zchunk == o.zchunk && t_block == o.t_block && xcd_order == o.xcd_order && ftile == o.ftile && autos == o.autos && fuse == o.fuse &&
            napplied == o.napplied;
   }
 };
@@ -273,9 +308,11 @@ extern "C" int gr_create(const gr_desc *d, gr_handle **out) {
   P.planes = P.nz + 2 * P.R;
   P.field_elems = (long long)P.pitch * P.rows * P.planes;
   h->lc.zchunk = 0;
+  h->lc.auto_variant = h->lc.auto_zchunk = true;
   {  // GIRIH_XCD_ORDER=1 or 2 starts from that workgroup order (the autotuner tries all three)
     const char *e = getenv("GIRIH_XCD_ORDER");
     h->lc.xcd_order = (e && (e[0] == '1' || e[0] == '2')) ? e[0] - '0' : 0;
+    h->lc.auto_order = h->lc.xcd_order == 0;
   }
   h->lc.t_block = d->t_block <= 0 ? 1 : d->t_block;  // 0: single sweeps until gr_autotune picks a depth
   if (h->lc.t_block > 1) {
@@ -532,7 +569,7 @@ extern "C" int gr_step(gr_handle *h, int napply) {
   }
   // graph mode: replay the launch sequence of an identical earlier call
   GraphKey key{napply, h->parity, h->lu[0], h->lu[1], h->lc.variant, h->lc.zchunk, h->lc.t_block, h->lc.xcd_order,
-               h->lc.ftile, fuse ? 1 : 0, -1};
+               h->lc.ftile, h->lc.auto_variant + 2 * h->lc.auto_zchunk + 4 * h->lc.auto_order, fuse ? 1 : 0, -1};
   if (h->src && h->napplied < h->nsrc) key.napplied = h->napplied;  // source pointers are baked in
   if (h->use_graph && napply > 0) {
     if (!(h->gexec && h->gkey == key)) {
@@ -587,6 +624,17 @@ static int round_chunk(const gr_handle *h, int tl, const LaunchCfg &lc, int roun
   return zc >= 2 * tl && zc < P.nz ? zc : 0;
 }
 
+// h's settings for fused passes of depth tl: chunks for one round of the CUs and, in FP32,
+// the XCD bands (512^3 kernel 5 FP32 1163 us a pass against 1261 in plain order, FP64 2457
+// against 2178) where the caller has set neither.
+static LaunchCfg fused_cfg(const gr_handle *h, int tl) {
+  LaunchCfg lc = h->lc;
+  if (tl != lc.t_block) lc.ftile = 0;  // a rest shallower than the configured depth
+  if (lc.auto_order) lc.xcd_order = h->P.dtype == GR_F32 && h->P.kernel != 0 ? 2 : 0;
+  if (lc.auto_zchunk || tl != lc.t_block) lc.zchunk = round_chunk(h, tl, lc, 1);
+  return lc;
+}
+
 // Launch napply applications of a first-order kernel as fused passes, the last of which
 // writes the field's last two levels (the U1/U2 pair a call leaves) into different
 // buffers, so that no single sweep is needed to make both exact: at 512^3, 20 kernel-5
@@ -624,11 +672,7 @@ static int enqueue_first_order(gr_handle *h, int napply, int *nlaunch) {
     const bool has_src = h->src && app < h->nsrc;
     const void *srcp = has_src ? (const char *)h->src + (size_t)app * es : nullptr;
     const long long sidx = has_src ? h->src_idx : -1;
-    LaunchCfg lc = h->lc;
-    if (ops[i] != lc.t_block) {  // a shallower pass: its own tile, and chunks for one round of the CUs
-      lc.ftile = 0;
-      if (ops[i] > 1) lc.zchunk = round_chunk(h, ops[i], lc, 1);
-    }
+    const LaunchCfg lc = ops[i] > 1 ? fused_cfg(h, ops[i]) : h->lc;
     const void *in = field_base(h, h->fbuf[x]);
     hipError_t e;
     if (i == m - 1) {
@@ -676,6 +720,7 @@ static int enqueue_apps(gr_handle *h, int napply, bool fuse, int *nlaunch) {
     // kernel 0 keeps (u^(n-1), u^n) exact after every pass; first-order kernels
     // keep the last application as a single sweep so U1 and U2 end exact.
     const int reserve = wave ? 0 : 1;
+    const LaunchCfg flc = fused_cfg(h, tl);
     while (napply - reserve - s >= tl) {
       const long long app = h->napplied + s;
       const bool has_src = h->src && app < h->nsrc;
@@ -687,13 +732,13 @@ static int enqueue_apps(gr_handle *h, int napply, bool fuse, int *nlaunch) {
         int sp[2];
         spare_ids(h, sp);
         e = tblock_pass(P, tl, ubase(h, w), ubase(h, r), field_base(h, h->fbuf[sp[0]]), field_base(h, h->fbuf[sp[1]]),
-                        srcp, sidx, h->lc, h->stream);
+                        srcp, sidx, flc, h->stream);
         h->parity ^= (tl & 1);
         h->lu[h->parity] = sp[0];      // written next: holds level tl-1
         h->lu[1 - h->parity] = sp[1];  // read next: level tl
       } else {
         const int pw = h->lu[w], pr = h->lu[r];
-        e = tblock_pass(P, tl, nullptr, ubase(h, r), nullptr, ubase(h, w), srcp, sidx, h->lc, h->stream);
+        e = tblock_pass(P, tl, nullptr, ubase(h, r), nullptr, ubase(h, w), srcp, sidx, flc, h->stream);
         h->parity ^= (tl & 1);
         h->lu[1 - h->parity] = pw;  // newest (level tl) is read next
         h->lu[h->parity] = pr;
@@ -759,17 +804,23 @@ extern "C" int gr_get_stats(gr_handle *h, gr_stats *out) {
   if (!h || !out) return fail(GR_EINVAL, "gr_get_stats: null argument");
   gr_stats s = h->stats;
   s.t_block = h->lc.t_block;
+  LaunchCfg lc = sweep_cfg(h->P.kernel, h->lc, h->P.nx, h->P.ny, h->P.nz);  // the settings in use
+  if (lc.t_block > 1) {
+    const LaunchCfg f = fused_cfg(h, lc.t_block);
+    lc.zchunk = f.zchunk;
+    lc.xcd_order = f.xcd_order;
+  }
   // the fused pass's tile when the configuration fuses steps, else the sweep's
-  if (h->lc.t_block < 2 || !fused_tile(h->P, h->lc.t_block, h->lc, &s.tile_x, &s.tile_y))
-    tile_of_variant(h->P.kernel, h->P.dtype, h->lc.variant, &s.tile_x, &s.tile_y);
-  s.zchunk = h->lc.zchunk;
+  if (lc.t_block < 2 || !fused_tile(h->P, lc.t_block, lc, &s.tile_x, &s.tile_y))
+    tile_of_variant(h->P.kernel, h->P.dtype, lc.variant, &s.tile_x, &s.tile_y);
+  s.zchunk = lc.zchunk;
   s.parity = h->parity;
   s.pitch_x = h->P.pitch;
   s.rows_y = h->P.rows;
   s.planes_z = h->P.planes;
   s.x_offset = h->P.xoff;
-  s.tile_variant = h->lc.variant;
-  s.xcd_order = h->lc.xcd_order;
+  s.tile_variant = lc.variant;
+  s.xcd_order = lc.xcd_order;
   *out = s;
   return GR_OK;
 }
@@ -780,8 +831,12 @@ extern "C" int gr_set_config(gr_handle *h, int variant, int zchunk, int t_block)
     if (variant >= num_tile_variants(h->P.kernel, h->P.dtype))
       return fail(GR_EINVAL, "gr_set_config: tile variant %d not available for kernel %d", variant, h->P.kernel);
     h->lc.variant = variant;
+    h->lc.auto_variant = false;
   }
-  if (zchunk >= 0) h->lc.zchunk = zchunk;
+  if (zchunk >= 0) {
+    h->lc.zchunk = zchunk;
+    h->lc.auto_zchunk = false;
+  }
   if (t_block >= 1) {
     if (t_block > 1) {
       int depths[8];
@@ -811,6 +866,7 @@ extern "C" int gr_set_xcd_order(gr_handle *h, int xcd_order) {
   if (!h) return fail(GR_EINVAL, "gr_set_xcd_order: null handle");
   if (xcd_order < 0 || xcd_order > 2) return fail(GR_EINVAL, "gr_set_xcd_order: 0, 1 or 2");
   h->lc.xcd_order = xcd_order;
+  h->lc.auto_order = false;
   return GR_OK;
 }
 
@@ -849,6 +905,8 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
     for (int zc : {16, 8})
       if (zc < nz) zchunks.push_back(zc);
   LaunchCfg best_lc = h->lc;
+  best_lc.auto_variant = best_lc.auto_zchunk = best_lc.auto_order = false;
+  const LaunchCfg lc0 = best_lc;
   float best_ms = 1e30f;
   std::vector<std::pair<float, LaunchCfg>> tried;  // sweep trials: time of `steps` sweeps
   // one untimed sweep, then n timed sweeps
@@ -882,7 +940,7 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
     float var_ms = 1e30f;
     for (int order = 0; order < 3 && !(order > 0 && var_ms > 1.4f * best_ms); ++order)
       for (int zc : {0, std::min(128, nz)}) {
-        LaunchCfg lc = h->lc;
+        LaunchCfg lc = lc0;
         lc.variant = var;
         lc.xcd_order = order;
         lc.zchunk = zc;
@@ -1083,7 +1141,8 @@ extern "C" int gr_sweep_dev(int kernel, int dtype, const int shape[3], int xb, i
   g.sz = (long long)shape[0] * shape[1];
   g.xb = xb; g.yb = yb; g.zb = zb; g.xe = xe; g.ye = ye; g.ze = ze;
   LaunchCfg lc;
-  hipError_t e = sweep_box(P, g, u, v, lc, nullptr);
+  lc.auto_variant = lc.auto_zchunk = lc.auto_order = true;
+  hipError_t e = sweep_box(P, g, u, v, sweep_cfg(kernel, lc, xe - xb, ye - yb, ze - zb), nullptr);
   if (e != hipSuccess) return fail(GR_EHIP, "gr_sweep_dev: %s", hipGetErrorString(e));
   HIP_TRY(hipStreamSynchronize(nullptr));
   return GR_OK;
