@@ -164,7 +164,6 @@ extern "C" int gr_download_roc2(gr_handle *h, const int ld[3], void *U3) {
   if (ld[0] < P.nx + 2 * P.R || ld[1] != P.ny + 2 * P.R || ld[2] != P.nz + 2 * P.R)
     return gr::set_error(GR_EINVAL, "gr_download_roc2: ldomain_shape does not fit the grid");
   const size_t es = gr::elem_size(P.dtype);
-  const size_t width = (size_t)(P.nx + 2 * P.R);
   hipStream_t s = gr_internal_stream(h);
   const void *src = P.roc2;
   void *tmp = nullptr;
@@ -183,11 +182,10 @@ extern "C" int gr_download_roc2(gr_handle *h, const int ld[3], void *U3) {
       src = (const char *)tmp + (size_t)P.xoff * es;
     }
   }
-  if (e == hipSuccess)
-    e = hipMemcpy2DAsync(U3, (size_t)ld[0] * es, src, (size_t)P.pitch * es, width * es, (size_t)P.rows * P.planes,
-                         hipMemcpyDeviceToHost, s);
+  int rc = GR_OK;
+  if (e == hipSuccess) rc = gr_internal_copy_field(h, ld, const_cast<void *>(src), U3, false);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (tmp) (void)hipFree(tmp);
   if (e != hipSuccess) return gr::set_errorf(GR_EHIP, "gr_download_roc2: %s", hipGetErrorString(e));
-  return GR_OK;
+  return rc;
 }

@@ -12,13 +12,18 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
+#include <sched.h>
+
 #include <algorithm>
+#include <atomic>
+#include <climits>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -103,7 +108,8 @@ void tile_of_variant(int kid, int dtype, int variant, int *tx, int *ty) {
 //    119, kernel 5 540 against 262).  Enough chunks for two 512-lane workgroups per CU
 //    (64^3 kernel 1 FP64: 54 us whole, 20 at 8 planes, 18 at 4), but not longer than the
 //    kernel gains from: 32 planes for kernel 0, whose chunks re-read 8 planes (512^3 FP32
-//    32 planes 486 us, 16 500), 16 for kernel 1 (512^3 FP32 247 us, 32 planes 248, 128
+//    32 planes 486 us, 16 500; on 64-wide tiles, more of which fit a CU, 16: 403 x 300 x
+//    219 FP32 119 us, 32 planes 135), 16 for kernel 1 (512^3 FP32 247 us, 32 planes 248, 128
 //    251), 4 where coefficient arrays are streamed (600 x 600 x 300 kernel 5 FP64 4 planes
 //    1490 us, 8 1534, 16 1558; 403 x 300 x 219 kernel 4 384, 405, 419);
 //  * tile: 128 x 16 of 1024 lanes (for kernel 0 with the operand prefetch) where it overhangs
@@ -122,7 +128,7 @@ LaunchCfg sweep_cfg(int kid, const LaunchCfg &lc, int nx, int ny, int nz) {
     int tx = 64, ty = 16;
     tile_of_variant(kid, 0, c.variant, &tx, &ty);
     const long long tiles = (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
-    const int most = kid == 0 ? 32 : kid == 1 ? 16 : 4;
+    const int most = kid == 0 ? (tx > 64 ? 32 : 16) : kid == 1 ? 16 : 4;
     c.zchunk = (int)std::min<long long>(most, std::max<long long>(4, tiles * nz / (tx > 64 ? 256 : 512)));
   }
   if (lc.auto_order) c.xcd_order = 2;
@@ -232,6 +238,9 @@ struct gr_handle {
   gr_stats stats{};
   int device = 0;
   int ncu = 1;         // compute units of the device
+  // pinned slots of the host-field copies (copy_rows), one event each
+  void *stage = nullptr;
+  hipEvent_t stage_ev[8] = {};
   // graph mode (gr_set_graph): the last captured step sequence and the state it leaves
   bool use_graph = false;
   hipGraphExec_t gexec = nullptr;
@@ -240,6 +249,7 @@ struct gr_handle {
 };
 
 static void drop_graph(gr_handle *h);
+static void free_stage(gr_handle *h);
 
 static void *field_base(const gr_handle *h, void *alloc) {
   return alloc ? (char *)alloc + (size_t)h->P.xoff * elem_size(h->P.dtype) : nullptr;
@@ -376,6 +386,7 @@ extern "C" int gr_destroy(gr_handle *h) {
   if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
   for (void *p : {h->fbuf[0], h->fbuf[1], h->fbuf[2], h->fbuf[3], h->alloc_roc2, h->alloc_coef, h->src, h->flag})
     if (p) (void)hipFree(p);
+  free_stage(h);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -388,18 +399,128 @@ __global__ void to_bf16_kernel(const float *src, __hip_bfloat16 *dst, long long 
   if (t < n) dst[t] = __float2bfloat16(src[t]);  // round to nearest even
 }
 
-// host girih layout <-> device layout: both store rows (k*nny + j) at a constant pitch
+// ------------------------------------------------------------------ host fields
+// host girih layout <-> device layout: both store rows (k*nny + j) at a constant pitch.
+// hipMemcpy2DAsync moves pageable pitched rows one by one (256 x 256 x 128 FP32, two
+// fields down: 495 ms, 0.15 GB/s).  Here a few host threads each take chunks of rows
+// through a pinned slot of their own: a kernel packs the rows into the slot (or unpacks
+// them from it) over the bus while the other threads copy theirs between slot and
+// array, which also spreads the page faults of fresh arrays.
+constexpr int kStageThreads = 8;                  // host threads and slots
+constexpr size_t kStageBytes = (size_t)2 << 20;   // one slot
+
+// rows of `width` words at `pitch` <-> rows at `width` (one wavefront per row)
+template <typename W, bool PACK>
+__global__ __launch_bounds__(256) void stage_rows_kernel(W *pitched, long long pitch, W *packed, int width, int nrows) {
+  const int row = blockIdx.x * 4 + threadIdx.x / 64;
+  if (row >= nrows) return;
+  W *a = pitched + row * pitch, *b = packed + (long long)row * width;
+  for (int i = threadIdx.x % 64; i < width; i += 64)
+    if (PACK)
+      b[i] = a[i];
+    else
+      a[i] = b[i];
+}
+
+template <typename W>
+static hipError_t stage_rows(bool pack, void *dev, long long pitch, void *slot, int width, int nrows, hipStream_t st) {
+  const dim3 grid((nrows + 3) / 4);
+  if (pack)
+    hipLaunchKernelGGL((stage_rows_kernel<W, true>), grid, dim3(256), 0, st, (W *)dev, pitch, (W *)slot, width, nrows);
+  else
+    hipLaunchKernelGGL((stage_rows_kernel<W, false>), grid, dim3(256), 0, st, (W *)dev, pitch, (W *)slot, width, nrows);
+  return hipGetLastError();
+}
+
+static void free_stage(gr_handle *h) {
+  for (hipEvent_t &e : h->stage_ev) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
+  }
+  if (h->stage) (void)hipHostFree(h->stage);
+  h->stage = nullptr;
+}
+
+// The handle's pinned slots, allocated on first use (false: not available).
+static bool ensure_stage(gr_handle *h) {
+  if (h->stage) return true;
+  bool ok = hipHostMalloc(&h->stage, kStageThreads * kStageBytes, hipHostMallocDefault) == hipSuccess;
+  if (!ok) h->stage = nullptr;
+  for (int i = 0; i < kStageThreads && ok; ++i)
+    ok = hipEventCreateWithFlags(&h->stage_ev[i], hipEventDisableTiming) == hipSuccess;
+  if (!ok) {
+    (void)hipGetLastError();
+    free_stage(h);
+  }
+  return ok;
+}
+
+// Host threads this process may use.
+static int host_threads() {
+  cpu_set_t set;
+  CPU_ZERO(&set);
+  return sched_getaffinity(0, sizeof(set), &set) == 0 ? std::max(1, CPU_COUNT(&set)) : 1;
+}
+
+static int copy_rows(gr_handle *h, char *dev, size_t dev_pitch, char *host, size_t host_pitch, size_t width, int nrows,
+                     size_t es, bool to_dev) {
+  const int per = (int)std::max<size_t>(1, kStageBytes / width);  // rows per chunk
+  const int nchunk = (nrows + per - 1) / per;
+  std::atomic<int> next{0}, err{(int)hipSuccess};
+  auto work = [&](int t) {
+    char *slot = (char *)h->stage + (size_t)t * kStageBytes;
+    hipError_t e = hipSetDevice(h->device);
+    bool busy = false;  // the slot is still being read by the unpacking kernel
+    for (int c; e == hipSuccess && err.load() == (int)hipSuccess && (c = next.fetch_add(1)) < nchunk;) {
+      const int r0 = c * per, n = std::min(per, nrows - r0);
+      char *d = dev + (size_t)r0 * dev_pitch, *u = host + (size_t)r0 * host_pitch;
+      if (busy) e = hipEventSynchronize(h->stage_ev[t]);
+      busy = false;
+      if (to_dev)
+        for (int r = 0; r < n; ++r) memcpy(slot + r * width, u + r * host_pitch, width);
+      if (e == hipSuccess)
+        e = es == 8 ? stage_rows<double>(!to_dev, d, (long long)(dev_pitch / 8), slot, (int)(width / 8), n, h->stream)
+                    : stage_rows<float>(!to_dev, d, (long long)(dev_pitch / 4), slot, (int)(width / 4), n, h->stream);
+      if (e == hipSuccess) e = hipEventRecord(h->stage_ev[t], h->stream);
+      if (e != hipSuccess) break;
+      busy = to_dev;
+      if (!to_dev && (e = hipEventSynchronize(h->stage_ev[t])) == hipSuccess)
+        for (int r = 0; r < n; ++r) memcpy(u + r * host_pitch, slot + r * width, width);
+    }
+    if (busy) (void)hipEventSynchronize(h->stage_ev[t]);
+    if (e != hipSuccess) err.store((int)e);
+  };
+  const int nt = std::min({kStageThreads, nchunk, host_threads()});
+  std::vector<std::thread> pool;
+  try {
+    for (int t = 1; t < nt; ++t) pool.emplace_back(work, t);
+  } catch (const std::exception &) {
+    // no more threads: those that run, and this one, take all chunks
+  }
+  work(0);
+  for (std::thread &t : pool) t.join();
+  const hipError_t e = (hipError_t)err.load();
+  return e == hipSuccess ? GR_OK : fail(GR_EHIP, "field copy: %s", hipGetErrorString(e));
+}
+
 static int copy_field(gr_handle *h, const int ld[3], void *dev_base, size_t dev_es, const void *host,
                       size_t host_es, bool to_dev) {
   const Problem &P = h->P;
-  const size_t width = (size_t)(P.nx + 2 * P.R);
+  const size_t width = (size_t)(P.nx + 2 * P.R) * host_es;
+  const size_t dpitch = (size_t)P.pitch * dev_es, hpitch = (size_t)ld[0] * host_es;
+  const size_t nrows = (size_t)P.rows * P.planes;
   if (dev_es != host_es) return fail(GR_EINVAL, "copy_field: element size mismatch");
+  // memory that host threads cannot touch (a device pointer), and rows longer than a slot go to the runtime's copy
+  hipPointerAttribute_t at{};
+  const bool dev_mem = hipPointerGetAttributes(&at, host) == hipSuccess && at.type == hipMemoryTypeDevice;
+  (void)hipGetLastError();
+  if (!dev_mem && width <= kStageBytes && nrows <= (size_t)INT_MAX && ensure_stage(h))
+    return copy_rows(h, (char *)dev_base, dpitch, (char *)const_cast<void *>(host), hpitch, width, (int)nrows, dev_es,
+                     to_dev);
   if (to_dev)
-    HIP_TRY(hipMemcpy2DAsync(dev_base, (size_t)P.pitch * dev_es, host, (size_t)ld[0] * host_es,
-                             width * host_es, (size_t)P.rows * P.planes, hipMemcpyHostToDevice, h->stream));
+    HIP_TRY(hipMemcpy2DAsync(dev_base, dpitch, host, hpitch, width, nrows, hipMemcpyHostToDevice, h->stream));
   else
-    HIP_TRY(hipMemcpy2DAsync((void *)host, (size_t)ld[0] * host_es, dev_base, (size_t)P.pitch * dev_es,
-                             width * host_es, (size_t)P.rows * P.planes, hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipMemcpy2DAsync((void *)host, hpitch, dev_base, dpitch, width, nrows, hipMemcpyDeviceToHost, h->stream));
   return GR_OK;
 }
 
@@ -1608,6 +1729,10 @@ void gr_internal_fused_advance(gr_handle *h, int npasses, int napply, double ms)
   h->stats.last_ms = ms;
   h->stats.last_updates = (int64_t)napply * h->P.nx * h->P.ny * h->P.nz;
   h->stats.last_launches = npasses + (napply - 2 * npasses);
+}
+int gr_internal_copy_field(gr_handle *h, const int ld[3], void *dev_base, void *host, bool to_dev) {
+  const size_t es = elem_size(h->P.dtype);
+  return copy_field(h, ld, dev_base, es, host, es, to_dev);
 }
 void gr_internal_advance(gr_handle *h, int napply, double ms) {
   h->parity ^= napply & 1;
