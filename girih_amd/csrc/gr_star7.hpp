@@ -20,6 +20,10 @@
 //   * kernel 5's coefficients of a plane are loaded one step before level 1 needs
 //     them and then stay in the lane's registers while the plane passes through the
 //     levels (one per step), so they are read from memory once;
+//   * the input is loaded PD planes ahead: kernel 1's plane step (0.3-0.8 us) is shorter
+//     than the latency of a load from HBM (512^3 with PD 2 against 1: FP32 depth 4 1694
+//     against 1472 GLUP/s, FP64 944 against 812); kernel 5, whose steps stream eight
+//     arrays, gains nothing;
 //   * the x margin is a whole number of slots and covers the input's ring, so only
 //     the ring rows above and below the region are loaded apart;
 //   * the plane loop is unrolled by UN steps, so queue (mod 3), LDS (mod 2) and
@@ -119,7 +123,8 @@ struct Star7 {
   static_assert(TX % P == 0 && UN % 6 == 0 && (NC == 0 || UN % TL == 0), "tile and unroll");
 };
 
-template <typename T, typename C, int KID, int TL, int TX, int TY, int NT, int P, bool STRM, bool GEN>
+template <typename T, typename C, int KID, int TL, int TX, int TY, int NT, int P, int PD, bool STRM,
+          bool GEN>
 __global__ __launch_bounds__(NT) void star7_tb_kernel(const S7Args<T, C> a) {
   using G = Star7<T, C, KID, TL, TX, TY, NT, P>;
   constexpr int W = G::W, H = G::H, WS = G::WS, NS = G::NS, NR = G::NR, NC = G::NC, UN = G::UN;
@@ -205,20 +210,22 @@ __global__ __launch_bounds__(NT) void star7_tb_kernel(const S7Args<T, C> a) {
   };
 
   const int kfirst = zs - TL, kend = ze + TL;  // step k: the input's plane k enters; level t computes k - t
-  T nv[NS][P], hv[NR][P];
-  auto fetch = [&](int k) {  // input plane k, the ring rows of plane k - 1, coefficients of plane k - 1
+  // input planes in flight: plane k's slots and the ring rows of plane k - 1 in k mod PD
+  T nv[PD][NS][P], hv[PD][NR][P];
+  auto fetch = [&](int k, int slot) {  // input plane k and the ring rows of plane k - 1
     const T *vp = yplane(k), *hp = yplane(k - 1);
 #pragma unroll
-    for (int j = 0; j < NS; ++j) ld_slot<T, P>(vp, off[j], nv[j]);
+    for (int j = 0; j < NS; ++j) ld_slot<T, P>(vp, off[j], nv[slot][j]);
 #pragma unroll
     for (int s = 0; s < NR; ++s)
-      if (rw[s]) ld_slot<T, P>(hp, roff[s], hv[s]);
-    if constexpr (NC > 0) {
-#pragma unroll
-      for (int j = 0; j < NS; ++j) ld_coefs(k - 1, j, nc[j]);
-    }
+      if (rw[s]) ld_slot<T, P>(hp, roff[s], hv[slot][s]);
   };
-  fetch(kfirst);
+#pragma unroll
+  for (int i = 0; i < PD; ++i) fetch(kfirst + i, i);
+  if constexpr (NC > 0) {
+#pragma unroll
+    for (int j = 0; j < NS; ++j) ld_coefs(kfirst - 1, j, nc[j]);
+  }
 
   auto put = [&](T *z, int p, int j, const T (&val)[P]) {  // the slot's output cells of plane p
     T *zp = z + (long long)p * a.sz;
@@ -242,7 +249,7 @@ __global__ __launch_bounds__(NT) void star7_tb_kernel(const S7Args<T, C> a) {
 #pragma unroll
     for (int j = 0; j < NS; ++j)
 #pragma unroll
-      for (int e = 0; e < P; ++e) q[0][j][qs][e] = nv[j][e];
+      for (int e = 0; e < P; ++e) q[0][j][qs][e] = nv[ph % PD][j][e];
     {
       T *L0 = lds[0][bs];
 #pragma unroll
@@ -250,7 +257,7 @@ __global__ __launch_bounds__(NT) void star7_tb_kernel(const S7Args<T, C> a) {
         st_slot<T, P>(L0 + lo[j] + W + PAD, q[0][j][qm1]);
 #pragma unroll
       for (int s = 0; s < NR; ++s)
-        if (rw[s]) st_slot<T, P>(L0 + rl[s], hv[s]);
+        if (rw[s]) st_slot<T, P>(L0 + rl[s], hv[ph % PD][s]);
     }
     if constexpr (NC > 0) {
 #pragma unroll
@@ -272,7 +279,11 @@ __global__ __launch_bounds__(NT) void star7_tb_kernel(const S7Args<T, C> a) {
 #pragma unroll
             for (int e = 0; e < CP; ++e) asm("" : "+v"(cs[t][j][m][e]));
     }
-    fetch(k + 1);
+    fetch(k + PD, ph % PD);
+    if constexpr (NC > 0) {
+#pragma unroll
+      for (int j = 0; j < NS; ++j) ld_coefs(k, j, nc[j]);  // level 1's next centre plane
+    }
     __syncthreads();
 
 #pragma unroll

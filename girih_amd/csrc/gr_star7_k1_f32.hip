@@ -7,29 +7,32 @@
 namespace gr {
 
 // A pass is bound by the vector ALU (11 instructions per computed cell, 10 of them the
-// stencil) and by the LDS reads behind each barrier, not by memory, so a tile trades the
-// margins it computes twice (1.33x the tile at 128 x 24, depth 4) against two
-// workgroups per CU, which cover each other's barriers.  512^3, one box, GLUP/s, against
-// one-cell lanes (1029-1179 at depth 4):
-//   depth 2: 128 x 32 1020, 128 x 16 1066 (4.3 TB/s);   depth 3: 128 x 16 1496, 64 x 16 1113;
-//   depth 4: 128 x 24 1472, 128 x 16 1279, 64 x 16 1230;  depth 5: 128 x 16 1597 (14
-//   wavefronts x 4 cells), 1394 with 2 cells per lane;  depth 6: 64 x 20 1099.
+// stencil; 86% busy at depth 5) and by the LDS reads behind each barrier, not by memory,
+// so a tile trades the margins it computes twice (1.33x the tile at 128 x 24, depth 4)
+// against two workgroups per CU, which cover each other's barriers.  512^3, one box,
+// GLUP/s, against one-cell lanes (1029-1179 at depth 4); in parentheses with the input
+// loaded one plane ahead instead of two:
+//   depth 2: 128 x 32 1280 (1020), 128 x 16 1231 (1066);
+//   depth 3: 128 x 16 1624 (1478), 64 x 16 1352 (1113);
+//   depth 4: 128 x 24 1714 three planes ahead, 1694 two (1472), 128 x 16 1690 (1279),
+//     64 x 16 1557 (1230);
+//   depth 5: 128 x 16 1663 (1597; 1394 with 2 cells per lane);  depth 6: 64 x 20 1150 (1099).
 // The 64-wide tiles are for grids that 128-wide tiles would mostly overhang.
 template <bool STRM>
 static hipError_t k1_dispatch(int tl, int tile, const S7Args<float, float> &a, hipStream_t st) {
   switch (tl) {
     case 2:
-      if (tile == 1) return launch_s7<float, float, 1, 2, 128, 16, 704, 2, STRM>(a, st);
-      return launch_s7<float, float, 1, 2, 128, 32, 832, 2, STRM>(a, st);
+      if (tile == 1) return launch_s7<float, float, 1, 2, 128, 16, 704, 2, 2, STRM>(a, st);
+      return launch_s7<float, float, 1, 2, 128, 32, 832, 2, 2, STRM>(a, st);
     case 3:
-      if (tile == 1) return launch_s7<float, float, 1, 3, 64, 16, 384, 2, STRM>(a, st);
-      return launch_s7<float, float, 1, 3, 128, 16, 704, 2, STRM>(a, st);
+      if (tile == 1) return launch_s7<float, float, 1, 3, 64, 16, 384, 2, 2, STRM>(a, st);
+      return launch_s7<float, float, 1, 3, 128, 16, 704, 2, 2, STRM>(a, st);
     case 4:
-      if (tile == 1) return launch_s7<float, float, 1, 4, 128, 24, 1024, 4, STRM>(a, st);
-      if (tile == 2) return launch_s7<float, float, 1, 4, 64, 16, 448, 4, STRM>(a, st);
-      return launch_s7<float, float, 1, 4, 128, 16, 768, 4, STRM>(a, st);
-    case 5: return launch_s7<float, float, 1, 5, 128, 16, 896, 4, STRM>(a, st);
-    case 6: return launch_s7<float, float, 1, 6, 64, 20, 640, 4, STRM>(a, st);
+      if (tile == 1) return launch_s7<float, float, 1, 4, 128, 24, 1024, 4, 3, STRM>(a, st);
+      if (tile == 2) return launch_s7<float, float, 1, 4, 64, 16, 448, 4, 2, STRM>(a, st);
+      return launch_s7<float, float, 1, 4, 128, 16, 768, 2, 2, STRM>(a, st);
+    case 5: return launch_s7<float, float, 1, 5, 128, 16, 896, 4, 2, STRM>(a, st);
+    case 6: return launch_s7<float, float, 1, 6, 64, 20, 640, 4, 2, STRM>(a, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -7,22 +7,23 @@
 namespace gr {
 
 // Two cells per lane (16-byte accesses).  512^3, one box, GLUP/s, against one-cell lanes
-// (557-640 at depth 3): depth 2: 64 x 16 559 (three workgroups per CU), 128 x 16 568;
-// depth 3: 64 x 16 798 (two per CU; 4.7 TB/s), 64 x 24 666, 128 x 8 472; depth 4:
-// 64 x 22 810, 64 x 16 703; depth 5: 64 x 14 693; depth 6: 64 x 8 569.  128^3 in the
-// caches, 8-plane chunks: depth 3 at 64 x 16 412 (before 294), 4 at 64 x 16 395.
+// (557-640 at depth 3); in parentheses with the input loaded one plane ahead instead of
+// two: depth 2: 64 x 16 652 (559; three workgroups per CU), 128 x 16 699 (568); depth 3:
+// 64 x 16 899 (798; two per CU, 4.7 TB/s), 64 x 24 666, 128 x 8 472; depth 4: 64 x 22 944
+// (812), 64 x 16 839 (703); depth 5: 64 x 14 685 (693); depth 6: 64 x 8 556 (569).  128^3
+// in the caches, 8-plane chunks: depth 3 at 64 x 16 432 (412; before 294), 4 at 64 x 16 413.
 template <bool STRM>
 static hipError_t k1_dispatch(int tl, int tile, const S7Args<double, double> &a, hipStream_t st) {
   switch (tl) {
     case 2:
-      if (tile == 1) return launch_s7<double, double, 1, 2, 128, 16, 640, 2, STRM>(a, st);
-      return launch_s7<double, double, 1, 2, 64, 16, 640, 2, STRM>(a, st);
-    case 3: return launch_s7<double, double, 1, 3, 64, 16, 768, 2, STRM>(a, st);
+      if (tile == 1) return launch_s7<double, double, 1, 2, 128, 16, 640, 2, 2, STRM>(a, st);
+      return launch_s7<double, double, 1, 2, 64, 16, 640, 2, 2, STRM>(a, st);
+    case 3: return launch_s7<double, double, 1, 3, 64, 16, 768, 2, 2, STRM>(a, st);
     case 4:
-      if (tile == 1) return launch_s7<double, double, 1, 4, 64, 22, 1024, 2, STRM>(a, st);
-      return launch_s7<double, double, 1, 4, 64, 16, 832, 2, STRM>(a, st);
-    case 5: return launch_s7<double, double, 1, 5, 64, 14, 1024, 2, STRM>(a, st);
-    case 6: return launch_s7<double, double, 1, 6, 64, 8, 768, 2, STRM>(a, st);
+      if (tile == 1) return launch_s7<double, double, 1, 4, 64, 22, 1024, 2, 2, STRM>(a, st);
+      return launch_s7<double, double, 1, 4, 64, 16, 832, 2, 2, STRM>(a, st);
+    case 5: return launch_s7<double, double, 1, 5, 64, 14, 1024, 2, 1, STRM>(a, st);
+    case 6: return launch_s7<double, double, 1, 6, 64, 8, 768, 2, 1, STRM>(a, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -28,22 +28,22 @@ template <typename T, typename C>
 static hipError_t k5_dispatch(int tl, int tile, const S7Args<T, C> &a, hipStream_t st) {
   constexpr bool B16 = std::is_same<C, __hip_bfloat16>::value;
   if constexpr (B16) {
-    if (tl == 2) return launch_s7<T, C, 5, 2, 64, 32, 640, 4, false>(a, st);
+    if (tl == 2) return launch_s7<T, C, 5, 2, 64, 32, 640, 4, 1, false>(a, st);
     if (tl == 4) {
-      if (tile == 1) return launch_s7<T, C, 5, 4, 128, 16, 768, 4, false>(a, st);
-      if (tile == 2) return launch_s7<T, C, 5, 4, 64, 16, 832, 2, false>(a, st);
-      return launch_s7<T, C, 5, 4, 64, 32, 704, 4, false>(a, st);
+      if (tile == 1) return launch_s7<T, C, 5, 4, 128, 16, 768, 4, 1, false>(a, st);
+      if (tile == 2) return launch_s7<T, C, 5, 4, 64, 16, 832, 2, 1, false>(a, st);
+      return launch_s7<T, C, 5, 4, 64, 32, 704, 4, 1, false>(a, st);
     }
-    if (tl == 6) return launch_s7<T, C, 5, 6, 64, 16, 1024, 2, false>(a, st);
+    if (tl == 6) return launch_s7<T, C, 5, 6, 64, 16, 1024, 2, 1, false>(a, st);
   } else if constexpr (sizeof(T) == 4) {
     if (tl == 2) {
-      if (tile == 1) return launch_s7<T, C, 5, 2, 128, 16, 704, 4, false>(a, st);
-      return launch_s7<T, C, 5, 2, 64, 32, 640, 2, false>(a, st);
+      if (tile == 1) return launch_s7<T, C, 5, 2, 128, 16, 704, 4, 1, false>(a, st);
+      return launch_s7<T, C, 5, 2, 64, 32, 640, 2, 1, false>(a, st);
     }
-    if (tl == 4) return launch_s7<T, C, 5, 4, 64, 16, 448, 4, false>(a, st);
+    if (tl == 4) return launch_s7<T, C, 5, 4, 64, 16, 448, 4, 1, false>(a, st);
   } else {
-    if (tl == 2) return launch_s7<T, C, 5, 2, 64, 16, 704, 2, false>(a, st);
-    if (tl == 4) return launch_s7<T, C, 5, 4, 64, 8, 512, 2, false>(a, st);
+    if (tl == 2) return launch_s7<T, C, 5, 2, 64, 16, 704, 2, 1, false>(a, st);
+    if (tl == 4) return launch_s7<T, C, 5, 4, 64, 8, 512, 2, 1, false>(a, st);
   }
   return hipErrorInvalidValue;
 }

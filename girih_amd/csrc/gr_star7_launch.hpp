@@ -4,7 +4,7 @@
 
 namespace gr {
 
-template <typename T, typename C, int KID, int TL, int TX, int TY, int NT, int P, bool STRM>
+template <typename T, typename C, int KID, int TL, int TX, int TY, int NT, int P, int PD, bool STRM>
 static hipError_t launch_s7(S7Args<T, C> a, hipStream_t st) {
   if (g_fused_tile_probe) {
     g_fused_tile_probe[0] = TX;
@@ -17,9 +17,9 @@ static hipError_t launch_s7(S7Args<T, C> a, hipStream_t st) {
   a.nzc = (a.nz + a.zchunk - 1) / a.zchunk;
   const dim3 grid(a.tiles_x * a.tiles_y * a.nzc);
   if (a.src_k >= 0 || a.Z1)
-    hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, STRM, true>), grid, dim3(NT), 0, st, a);
+    hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, PD, STRM, true>), grid, dim3(NT), 0, st, a);
   else
-    hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, STRM, false>), grid, dim3(NT), 0, st, a);
+    hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, PD, STRM, false>), grid, dim3(NT), 0, st, a);
   return hipGetLastError();
 }
 
