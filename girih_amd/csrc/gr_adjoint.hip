@@ -17,9 +17,11 @@
 // a pointwise accumulation (differences in FP64, sum in the field type) with no
 // second stencil pass.
 //
-// The forward pass stores (x_{cK}, x_{cK+1}) every K applications; the backward
-// pass recomputes each segment's K states from its checkpoint into a buffer and
-// walks it backwards.  Memory: 2*ceil(nt/K) + 2 fields for the forward pass;
+// The forward pass keeps (x_{cK}, x_{cK+1}) every K applications, written by the sweeps
+// straight into the checkpoints' fields; the backward pass recomputes each segment's K
+// states from its checkpoint, read in place, into a buffer and walks it backwards, the
+// adjoint fields of the segments following each other in a ring (400^3 FP32, 100 steps,
+// checkpoints every 50: 71.4 -> 70.1 ms without the fields' copies).  Memory: 2*ceil(nt/K) + 2 fields for the forward pass;
 // the first backward pass adds 2K + 4 fields (the segment's states and adjoint
 // fields) and a dense accumulator, which takes a segment's gradient terms in one pass.
 #include <hip/hip_runtime.h>
@@ -70,7 +72,8 @@ __global__ void inject_kernel_same(T *nu, const T *roc2, long long sy, long long
 // fields xs + t * fstride; nu_{a+2} is field nus + (a - a0) * fstride.  The source
 // term applies at cell src_idx for steps a < nsrc.
 template <typename T>
-__global__ void grad_segment_kernel(T *g, const T *__restrict__ nus, const T *__restrict__ xs, long long fstride,
+__global__ void grad_segment_kernel(T *g, const T *__restrict__ nus, int nub, int nring, const T *__restrict__ x0,
+                                    const T *__restrict__ x1, const T *__restrict__ xs, long long fstride,
                                     long long sy, long long sz, int nx, int ny, int R, int nsteps, const T *src,
                                     long long src_idx, int a0, int nsrc) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y, k = blockIdx.z;
@@ -79,8 +82,10 @@ __global__ void grad_segment_kernel(T *g, const T *__restrict__ nus, const T *__
   T &gc = g[((long long)k * ny + j) * nx + i];
   T acc = gc;
   const bool at_src = src && o == src_idx;
-  double x2 = (double)xs[(long long)(nsteps + 1) * fstride + o];  // x_{a+2} for a = a1 - 1
-  double x1 = (double)xs[(long long)nsteps * fstride + o];
+  auto xf = [&](int t) { return t == 0 ? x0 : t == 1 ? x1 : xs + (long long)t * fstride; };
+  auto nuf = [&](int t) { return nus + (long long)(nub + t < nring ? nub + t : nub + t - nring) * fstride; };
+  double xa2 = (double)xf(nsteps + 1)[o];  // x_{a+2} for a = a1 - 1
+  double xa1 = (double)xf(nsteps)[o];
   // the loads of QB steps are issued together (each cell's terms are still added one
   // step at a time, in the walk's order)
   constexpr int QB = 8;
@@ -89,19 +94,19 @@ __global__ void grad_segment_kernel(T *g, const T *__restrict__ nus, const T *__
 #pragma unroll
     for (int q = 0; q < QB; ++q)
       if (t0 - q >= 0) {
-        xq[q] = __builtin_nontemporal_load(xs + (long long)(t0 - q) * fstride + o);
-        nq[q] = __builtin_nontemporal_load(nus + (long long)(t0 - q) * fstride + o);
+        xq[q] = __builtin_nontemporal_load(xf(t0 - q) + o);
+        nq[q] = __builtin_nontemporal_load(nuf(t0 - q) + o);
       }
 #pragma unroll
     for (int q = 0; q < QB; ++q)
       if (t0 - q >= 0) {
         const int t = t0 - q;
-        const double x0 = (double)xq[q];
-        double d = (x2 - x1) - (x1 - x0);
+        const double xa0 = (double)xq[q];
+        double d = (xa2 - xa1) - (xa1 - xa0);
         if (at_src && a0 + t < nsrc) d = d - (double)src[a0 + t];
         acc = (T)((double)acc + (double)nq[q] * d);
-        x2 = x1;
-        x1 = x0;
+        xa2 = xa1;
+        xa1 = xa0;
       }
   }
   gc = acc;
@@ -158,9 +163,9 @@ struct gr_shot {
   double dt_over_h = 0;
   std::vector<void *> allocs;  // everything below lives in these
   std::vector<void *> ck;      // 2*nck checkpoint fields (x_{cK}, x_{cK+1})
-  void *seg = nullptr;         // ckpt+2 recompute fields x_{a0} .. x_{a1+1}, contiguous
-  void *nus = nullptr;         // ckpt+2 adjoint fields nu_{a0+2} .. nu_{a1+3}, contiguous
-  void *x[2] = {nullptr, nullptr};  // forward ping-pong
+  void *seg = nullptr;         // ckpt+2 recompute fields; x_{a0+t} in field t for t >= 2
+  void *nus = nullptr;         // ckpt+2 adjoint fields nu_{a0+2} .. nu_{a1+3}, a ring over the segments
+  void *x[2] = {nullptr, nullptr};  // forward states between checkpoints
   void *g = nullptr;  // gradient accumulator, field type, dense interior
   bool have_forward = false;
 };
@@ -201,7 +206,8 @@ hipError_t inject_any(const Problem &P, void *nu, int rec_k, const void *res, hi
 }
 
 // the accumulation of one segment's nsteps steps starting at a0 (grad_segment_kernel)
-hipError_t grad_segment(gr_handle *h, void *g, const void *nus, const void *xs, int nsteps, int a0, hipStream_t st) {
+hipError_t grad_segment(gr_handle *h, void *g, const void *nus, int nub, int nring, const void *x0, const void *x1,
+                        const void *xs, int nsteps, int a0, hipStream_t st) {
   const Problem &P = gr_internal_problem(h);
   const long long sz = (long long)P.pitch * P.rows;
   const dim3 grid((P.nx + 255) / 256, P.ny, P.nz);
@@ -213,13 +219,13 @@ hipError_t grad_segment(gr_handle *h, void *g, const void *nus, const void *xs, 
     sidx = -1;
   }
   if (P.dtype == GR_F64)
-    hipLaunchKernelGGL(grad_segment_kernel<double>, grid, dim3(256), 0, st, (double *)g, (const double *)nus,
-                       (const double *)xs, (long long)P.field_elems, (long long)P.pitch, sz, P.nx, P.ny, P.R, nsteps,
-                       (const double *)src, sidx, a0, nsrc);
+    hipLaunchKernelGGL(grad_segment_kernel<double>, grid, dim3(256), 0, st, (double *)g, (const double *)nus, nub,
+                       nring, (const double *)x0, (const double *)x1, (const double *)xs, (long long)P.field_elems,
+                       (long long)P.pitch, sz, P.nx, P.ny, P.R, nsteps, (const double *)src, sidx, a0, nsrc);
   else
-    hipLaunchKernelGGL(grad_segment_kernel<float>, grid, dim3(256), 0, st, (float *)g, (const float *)nus,
-                       (const float *)xs, (long long)P.field_elems, (long long)P.pitch, sz, P.nx, P.ny, P.R, nsteps,
-                       (const float *)src, sidx, a0, nsrc);
+    hipLaunchKernelGGL(grad_segment_kernel<float>, grid, dim3(256), 0, st, (float *)g, (const float *)nus, nub,
+                       nring, (const float *)x0, (const float *)x1, (const float *)xs, (long long)P.field_elems,
+                       (long long)P.pitch, sz, P.nx, P.ny, P.R, nsteps, (const float *)src, sidx, a0, nsrc);
   return hipGetLastError();
 }
 
@@ -319,20 +325,22 @@ extern "C" int gr_shot_forward(gr_shot *s, void *rec_dev) {
   const size_t fbytes = (size_t)P.field_elems * gr::elem_size(P.dtype);
   const size_t plane = (size_t)P.nx * P.ny * gr::elem_size(P.dtype);
   hipError_t e = hipSuccess;
-  for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipMemsetAsync(s->x[i], 0, fbytes, st);
-  void *prev = s->x[0], *cur = s->x[1];  // x_a, x_{a+1}
+  // x_0 = x_1 = 0 are the first checkpoint (zero since gr_shot_create); a sweep writes a
+  // checkpoint's state straight into its field, and any other state into the scratch
+  // field that x_{a+1} is not in (x_a's own where that is in scratch)
+  void *prev = s->ck[0], *cur = s->ck[1];  // x_a, x_{a+1}
   for (int a = 0; a < s->nt && e == hipSuccess; ++a) {
-    if (a % s->ckpt == 0) {
-      const int c = a / s->ckpt;
-      e = hipMemcpyAsync(s->ck[2 * c], prev, fbytes, hipMemcpyDeviceToDevice, st);
-      if (e == hipSuccess) e = hipMemcpyAsync(s->ck[2 * c + 1], cur, fbytes, hipMemcpyDeviceToDevice, st);
-      if (e != hipSuccess) break;
-    }
+    const int c0 = (a + 2) / s->ckpt, c1 = (a + 1) / s->ckpt;  // x_{a+2} opens checkpoint c0, or is c1's second
+    const bool first = (a + 2) % s->ckpt == 0 && c0 < s->nck, second = (a + 1) % s->ckpt == 0 && c1 < s->nck;
+    void *out = first ? s->ck[2 * c0] : second ? s->ck[2 * c1 + 1] : cur == s->x[0] ? s->x[1] : s->x[0];
     long long sidx = -1;
     const void *sv = src_of(h, a, &sidx);
-    e = gr::sweep_fields(P, fbase(P, prev), fbase(P, cur), sv, sidx, lc, st);  // prev <- x_{a+2}
-    if (e == hipSuccess) e = record_any(P, fbase(P, prev), s->rec_k, (char *)rec_dev + (size_t)a * plane, st);
-    std::swap(prev, cur);
+    e = gr::sweep_fields(P, fbase(P, out), fbase(P, cur), sv, sidx, lc, st, out == prev ? nullptr : fbase(P, prev));
+    if (e == hipSuccess) e = record_any(P, fbase(P, out), s->rec_k, (char *)rec_dev + (size_t)a * plane, st);
+    if (first && second && e == hipSuccess)  // checkpoints after every step: the state belongs to two
+      e = hipMemcpyAsync(s->ck[2 * c1 + 1], out, fbytes, hipMemcpyDeviceToDevice, st);
+    prev = cur;
+    cur = out;
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) return shot_fail(e, "gr_shot_forward");
@@ -409,8 +417,8 @@ extern "C" int gr_shot_adjoint(gr_shot *s, const void *res_dev, void *grad_dev) 
       return gr::set_errorf(GR_ENOMEM, "gr_shot_adjoint: device allocation failed: %s", hipGetErrorString(e));
     }
   }
-  auto segf = [&](int t) { return (void *)((char *)s->seg + (size_t)t * fbytes); };  // x_{a0+t}
-  auto nuf = [&](int t) { return (void *)((char *)s->nus + (size_t)t * fbytes); };   // nu_{a0+2+t}
+  const int nring = nslot;
+  int nub = 0;  // ring field of the segment's nu_{a0+2}
   if (e == hipSuccess) {
     if (P.dtype == GR_F64)
       hipLaunchKernelGGL(zero_kernel<double>, dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0, st, (double *)s->g,
@@ -422,32 +430,32 @@ extern "C" int gr_shot_adjoint(gr_shot *s, const void *res_dev, void *grad_dev) 
   }
   for (int c = s->nck - 1; c >= 0 && e == hipSuccess; --c) {
     const int a0 = c * s->ckpt, a1 = std::min(a0 + s->ckpt, s->nt), K = a1 - a0;
-    // recompute x_{a0} .. x_{a1+1} into seg slots 0 .. K+1
-    e = hipMemcpyAsync(segf(0), s->ck[2 * c], fbytes, hipMemcpyDeviceToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(segf(1), s->ck[2 * c + 1], fbytes, hipMemcpyDeviceToDevice, st);
-    for (int a = a0; a < a1 && e == hipSuccess; ++a) {
+    auto xf = [&](int t) {  // x_{a0+t}: the checkpoint, then the recomputed states
+      return fbase(P, t < 2 ? s->ck[2 * c + t] : (void *)((char *)s->seg + (size_t)t * fbytes));
+    };
+    auto nuf = [&](int t) {  // nu_{a0+2+t}
+      return fbase(P, (char *)s->nus + (size_t)((nub + t) % nring) * fbytes);
+    };
+    for (int a = a0; a < a1 && e == hipSuccess; ++a) {  // recompute x_{a0+2} .. x_{a1+1}
       const int t = a - a0 + 2;
       long long sidx = -1;
       const void *sv = src_of(h, a, &sidx);
-      e = gr::sweep_fields(P, fbase(P, segf(t)), fbase(P, segf(t - 1)), sv, sidx, lc, st, fbase(P, segf(t - 2)));
+      e = gr::sweep_fields(P, xf(t), xf(t - 1), sv, sidx, lc, st, xf(t - 2));
     }
-    // nu_{a1+2}, nu_{a1+3} into slots K, K+1: zero after the last step, else the two
-    // lowest of the later segment (its slots 0 and 1)
-    if (e == hipSuccess) {
-      if (c == s->nck - 1) {
-        e = hipMemsetAsync(nuf(K), 0, fbytes, st);
-        if (e == hipSuccess) e = hipMemsetAsync(nuf(K + 1), 0, fbytes, st);
-      } else {  // slot 1 first: with K = 1 slot 1 is also a destination
-        e = hipMemcpyAsync(nuf(K + 1), nuf(1), fbytes, hipMemcpyDeviceToDevice, st);
-        if (e == hipSuccess) e = hipMemcpyAsync(nuf(K), nuf(0), fbytes, hipMemcpyDeviceToDevice, st);
-      }
+    // nu_{a1+2} and nu_{a1+3} are zero after the last step, else the two lowest of the
+    // later segment, which this segment's ring position makes its fields K and K+1
+    if (c == s->nck - 1) {
+      for (int t = K; t < K + 2 && e == hipSuccess; ++t)
+        e = hipMemsetAsync((char *)s->nus + (size_t)((nub + t) % nring) * fbytes, 0, fbytes, st);
     }
-    for (int a = a1 - 1; a >= a0 && e == hipSuccess; --a) {  // nu_{a+2} <- f(nu_{a+3}, nu_{a+4})
+    for (int a = a1 - 1; a >= a0 && e == hipSuccess; --a) {  // nu_{a+2} <- f(nu_{a+3}, nu_{a+4}) + roc2 * residual
       const int t = a - a0;
-      e = gr::sweep_fields(P, fbase(P, nuf(t)), fbase(P, nuf(t + 1)), nullptr, -1, lc, st, fbase(P, nuf(t + 2)));
-      if (e == hipSuccess) e = inject_any(P, fbase(P, nuf(t)), s->rec_k, (const char *)res_dev + (size_t)a * plane, st);
+      e = gr::sweep_fields(P, nuf(t), nuf(t + 1), nullptr, -1, lc, st, nuf(t + 2));
+      if (e == hipSuccess) e = inject_any(P, nuf(t), s->rec_k, (const char *)res_dev + (size_t)a * plane, st);
     }
-    if (e == hipSuccess) e = grad_segment(h, s->g, fbase(P, nuf(0)), fbase(P, segf(0)), K, a0, st);
+    if (e == hipSuccess)
+      e = grad_segment(h, s->g, fbase(P, s->nus), nub, nring, xf(0), xf(1), fbase(P, s->seg), K, a0, st);
+    nub = (nub + nring - s->ckpt % nring) % nring;  // the earlier segment ends where this one begins
   }
   if (e == hipSuccess) {
     const double scale = -1.0 / (s->dt_over_h * s->dt_over_h);
