@@ -114,9 +114,11 @@ template <typename C, int BX, int BY, int RY, bool RING>
 __device__ __forceinline__ void step_items(const BatchDesc *__restrict__ d, int nprob, int nitems,
                                            unsigned long long *ctr, unsigned long long base, int step,
                                            typename SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX,
-                                                              true>::Lds &lds,
+                                                              true, false, false, true>::Lds &lds,
                                            int *sclaim) {
-  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true>;  // a step streams every problem
+  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true, false, false, true>;
+  // (a step streams every problem, and LATE: 16 problems of 192..512, 10 steps, 20.5 -> 19.9 ms;
+  // the single-grid sweeps lose 3% with it)
   const bool leader = threadIdx.x == 0 && threadIdx.y == 0;
   for (;;) {
     if (leader) {
@@ -167,7 +169,7 @@ template <typename C, int BX, int BY, int RY, bool RING>
 __global__ __launch_bounds__(64 * BX * BY) void batch_kernel(const BatchDesc *__restrict__ d, int nprob, int nitems,
                                                              unsigned long long *ctr, unsigned long long base,
                                                              int step) {
-  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true>;
+  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true, false, false, true>;
   __shared__ typename ST::Lds lds;
   __shared__ int sclaim[2];
   step_items<C, BX, BY, RY, RING>(d, nprob, nitems, ctr, base, step, lds, sclaim);
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(64 * BX * BY) void batch_run_kernel(const BatchDesc
                                                                  int nitems, unsigned long long *ctr, int napply,
                                                                  const RecDesc *__restrict__ rec, int nrec,
                                                                  int nrows) {
-  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true>;
+  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true, false, false, true>;
   __shared__ typename ST::Lds lds;
   __shared__ int sclaim[2];
   cooperative_groups::grid_group grid = cooperative_groups::this_grid();

@@ -253,8 +253,10 @@ struct Tile {
 // offset) instead of global loads; measured per case, see the launch code.
 // PF (kernel 0): the u^(n-1) and roc2 operands of plane k+1 are loaded while plane k
 // is computed, so their latency overlaps a whole plane instead of the LDS exchange.
+// LATE: a plane's rows are all computed before the source is added and any is stored
+// (one branch and one run of stores per plane instead of one per row).
 template <typename T, typename C, int KID, int BY, int RY, bool FAST, bool ROCS, bool RING, int ND, int BX = 1,
-          bool STRM = false, bool BUF = false, bool PF = false>
+          bool STRM = false, bool BUF = false, bool PF = false, bool LATE = false>
 struct SweepTile;
 
 // MINW > 0 asks the compiler for at least MINW waves per SIMD (caps VGPRs at 512/MINW).
@@ -279,7 +281,7 @@ void sweep_kernel(const SweepArgs<T, C> a) {
 // One tile of one sweep: the z-streaming body shared by the single-grid kernel
 // and the batched persistent kernel.
 template <typename T, typename C, int KID, int BY, int RY, bool FAST, bool ROCS, bool RING, int ND, int BX, bool STRM,
-          bool BUF, bool PF>
+          bool BUF, bool PF, bool LATE>
 struct SweepTile {
   static constexpr int R = kradius(KID);
   static constexpr int TX = 64 * BX, TY = BY * RY;
@@ -290,8 +292,8 @@ struct SweepTile {
 };
 
 template <typename T, typename C, int KID, int BY, int RY, bool FAST, bool ROCS, bool RING, int ND, int BX, bool STRM,
-          bool BUF, bool PF>
-__device__ __forceinline__ void SweepTile<T, C, KID, BY, RY, FAST, ROCS, RING, ND, BX, STRM, BUF, PF>::run(const SweepArgs<T, C> &a,
+          bool BUF, bool PF, bool LATE>
+__device__ __forceinline__ void SweepTile<T, C, KID, BY, RY, FAST, ROCS, RING, ND, BX, STRM, BUF, PF, LATE>::run(const SweepArgs<T, C> &a,
                                                                                    int tile_x, int tile_y, int zc,
                                                                                    Lds &lds) {
   constexpr int Q = 2 * R + 1;
@@ -462,6 +464,18 @@ __device__ __forceinline__ void SweepTile<T, C, KID, BY, RY, FAST, ROCS, RING, N
 
       T *__restrict__ uk = a.u + (long long)k * g.sz;
       const bool src_plane = a.src_k >= 0 && k == a.src_k;  // src_k = -1: no source
+      auto source = [&](int m, T &out) {
+        if (off[m] == (unsigned)a.src_off * (unsigned)sizeof(T)) out = out + *a.src;
+      };
+      auto put = [&](int m, T out) {
+        if (yout[m]) {
+          if constexpr (BUF)
+            bstore<STRM>(out, plane_rsrc(uk, pbytes), off[m]);
+          else
+            stb_stream<T, STRM>(uk, off[m], out);
+        }
+      };
+      T outv[RY];
 #pragma unroll
       for (int m = 0; m < RY; ++m) {
         const int ly = R + ty * RY + m, lx = R + tx;
@@ -497,13 +511,20 @@ __device__ __forceinline__ void SweepTile<T, C, KID, BY, RY, FAST, ROCS, RING, N
           out = cf[m][0] * v0 + cf[m][1] * xn(-1) + cf[m][2] * xn(1) + cf[m][3] * yn(-1) +
                 cf[m][4] * yn(1) + cf[m][5] * zq[0] + cf[m][6] * zq[2];
         }
-        if (src_plane && off[m] == (unsigned)a.src_off * (unsigned)sizeof(T)) out = out + *a.src;
-        if (yout[m]) {
-          if constexpr (BUF)
-            bstore<STRM>(out, plane_rsrc(uk, pbytes), off[m]);
-          else
-            stb_stream<T, STRM>(uk, off[m], out);
+        if constexpr (LATE) {
+          outv[m] = out;
+        } else {
+          if (src_plane) source(m, out);
+          put(m, out);
         }
+      }
+      if constexpr (LATE) {
+        if (src_plane) {
+#pragma unroll
+          for (int m = 0; m < RY; ++m) source(m, outv[m]);
+        }
+#pragma unroll
+        for (int m = 0; m < RY; ++m) put(m, outv[m]);
       }
 #pragma unroll
       for (int m = 0; m < RY; ++m) q[m][p] = nq[m];
