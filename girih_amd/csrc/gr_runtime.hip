@@ -734,15 +734,17 @@ extern "C" int gr_step(gr_handle *h, int napply) {
 }
 
 // The z chunk with which a pass of depth tl has at most `rounds` workgroups per CU, as
-// near to that as whole chunks allow (0: the whole z, or chunks shorter than 2*tl planes,
-// which would mostly compute each other's ghost planes).
+// near to that as whole chunks allow, but no chunk shorter than 2*tl planes: those would
+// mostly compute each other's ghost planes (0: the whole z).
 static int round_chunk(const gr_handle *h, int tl, const LaunchCfg &lc, int rounds) {
   const Problem &P = h->P;
   int tx = 0, ty = 0;
   if (!fused_tile(P, tl, lc, &tx, &ty)) return 0;
   const int ntile = ((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty);
-  const int nzc = rounds * h->ncu / ntile, zc = nzc > 0 ? (P.nz + nzc - 1) / nzc : 0;
-  return zc >= 2 * tl && zc < P.nz ? zc : 0;
+  const int nzc = rounds * h->ncu / ntile;
+  if (nzc < 1) return 0;
+  const int zc = std::max(2 * tl, (P.nz + nzc - 1) / nzc);
+  return zc < P.nz ? zc : 0;
 }
 
 // h's settings for fused passes of depth tl: chunks for one round of the CUs and, in FP32,
