@@ -110,15 +110,14 @@ __device__ __forceinline__ X uniform_load(const X *p) {
 
 // Claim and run the items of one step until the queue is empty.  `base` is the
 // counter value at which the step's claims start.
-template <typename C, int BX, int BY, int RY, bool RING>
+template <typename C, int BX, int BY, int RY, bool RING, bool LATE>
 __device__ __forceinline__ void step_items(const BatchDesc *__restrict__ d, int nprob, int nitems,
                                            unsigned long long *ctr, unsigned long long base, int step,
                                            typename SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX,
-                                                              true, false, false, true>::Lds &lds,
+                                                              true, false, false, LATE>::Lds &lds,
                                            int *sclaim) {
-  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true, false, false, true>;
-  // (a step streams every problem, and LATE: 16 problems of 192..512, 10 steps, 20.5 -> 19.9 ms;
-  // the single-grid sweeps lose 3% with it)
+  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true, false, false, LATE>;
+  // a step streams every problem
   const bool leader = threadIdx.x == 0 && threadIdx.y == 0;
   for (;;) {
     if (leader) {
@@ -165,14 +164,14 @@ __device__ __forceinline__ void step_items(const BatchDesc *__restrict__ d, int 
 }
 
 // One step per launch.
-template <typename C, int BX, int BY, int RY, bool RING>
+template <typename C, int BX, int BY, int RY, bool RING, bool LATE>
 __global__ __launch_bounds__(64 * BX * BY) void batch_kernel(const BatchDesc *__restrict__ d, int nprob, int nitems,
                                                              unsigned long long *ctr, unsigned long long base,
                                                              int step) {
-  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true, false, false, true>;
+  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true, false, false, LATE>;
   __shared__ typename ST::Lds lds;
   __shared__ int sclaim[2];
-  step_items<C, BX, BY, RY, RING>(d, nprob, nitems, ctr, base, step, lds, sclaim);
+  step_items<C, BX, BY, RY, RING, LATE>(d, nprob, nitems, ctr, base, step, lds, sclaim);
 }
 
 // Every step of a call in one cooperative launch: the workgroups run a step's
@@ -184,19 +183,19 @@ __global__ __launch_bounds__(64 * BX * BY) void batch_kernel(const BatchDesc *__
 // With receivers, step s's planes are recorded after its barrier, while step s+1
 // runs: step s+1 writes the other field of each pair, and the barrier after it
 // orders the recording before step s+2 overwrites the recorded field.
-template <typename C, int BX, int BY, int RY, bool RING>
+template <typename C, int BX, int BY, int RY, bool RING, bool LATE>
 __global__ __launch_bounds__(64 * BX * BY) void batch_run_kernel(const BatchDesc *__restrict__ d, int nprob,
                                                                  int nitems, unsigned long long *ctr, int napply,
                                                                  const RecDesc *__restrict__ rec, int nrec,
                                                                  int nrows) {
-  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true, false, false, true>;
+  using ST = SweepTile<float, C, 0, BY, RY, true, false, RING, kFastND, BX, true, false, false, LATE>;
   __shared__ typename ST::Lds lds;
   __shared__ int sclaim[2];
   cooperative_groups::grid_group grid = cooperative_groups::this_grid();
   const unsigned long long per = (unsigned long long)nitems + gridDim.x;
   const int lane = threadIdx.y * blockDim.x + threadIdx.x, nlanes = blockDim.x * blockDim.y;
   for (int s = 0; s < napply; ++s) {
-    step_items<C, BX, BY, RY, RING>(d + (size_t)(s & 1) * nprob, nprob, nitems, ctr, per * s, s, lds, sclaim);
+    step_items<C, BX, BY, RY, RING, LATE>(d + (size_t)(s & 1) * nprob, nprob, nitems, ctr, per * s, s, lds, sclaim);
     grid.sync();
     for (int row = blockIdx.x; row < nrows; row += gridDim.x)
       record_row(d + (size_t)(s & 1) * nprob, rec, nrec, row, s, lane, nlanes);
@@ -332,15 +331,22 @@ struct BatchVariant {
   batch_run_fn run32, runbf16;  // every step of a call in one cooperative launch
 };
 
-// tiles of 64*BX x BY*RY cells, 64*BX x BY lanes
-#define GR_BV(BX, BY, RY, RING)                                                                                   \
-  {                                                                                                              \
-    BX, BY, RY, RING, &batch_kernel<float, BX, BY, RY, RING>, &batch_kernel<__hip_bfloat16, BX, BY, RY, RING>,   \
-        &batch_run_kernel<float, BX, BY, RY, RING>, &batch_run_kernel<__hip_bfloat16, BX, BY, RY, RING>         \
+// tiles of 64*BX x BY*RY cells, 64*BX x BY lanes.  LATE (SweepTile) where it measured faster
+// (16 problems of 192..512 with bf16 roc2, 64-plane items, us per step with / without):
+// 64 x 32 2149 / 2398, its ring 1993 / 2042, 64 x 16 ring of 256 lanes 2064 / 2149, 128 x 16
+// ring of 1024 lanes 2106 / 2164; but 64 x 16 of 256 lanes 2830 / 2113, its ring of 512
+// lanes 2111 / 2072, 128 x 16 ring of 512 lanes 2299 / 2056.
+#define GR_BV(BX, BY, RY, RING, LATE)                                                        \
+  {                                                                                          \
+    BX, BY, RY, RING, &batch_kernel<float, BX, BY, RY, RING, LATE>,                          \
+        &batch_kernel<__hip_bfloat16, BX, BY, RY, RING, LATE>,                               \
+        &batch_run_kernel<float, BX, BY, RY, RING, LATE>,                                    \
+        &batch_run_kernel<__hip_bfloat16, BX, BY, RY, RING, LATE>                            \
   }
-const BatchVariant kVariants[] = {GR_BV(1, 8, 4, false), GR_BV(1, 8, 4, true), GR_BV(1, 4, 4, false),
-                                  GR_BV(1, 8, 2, true),  GR_BV(1, 4, 4, true), GR_BV(2, 8, 2, true),
-                                  GR_BV(2, 4, 4, true)};
+const BatchVariant kVariants[] = {GR_BV(1, 8, 4, false, true), GR_BV(1, 8, 4, true, true),
+                                  GR_BV(1, 4, 4, false, false), GR_BV(1, 8, 2, true, false),
+                                  GR_BV(1, 4, 4, true, true),  GR_BV(2, 8, 2, true, true),
+                                  GR_BV(2, 4, 4, true, false)};
 #undef GR_BV
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
@@ -893,7 +899,9 @@ extern "C" int gr_batch_autotune(gr_batch *b, int steps, int use_graph, int *var
     if (!gr_internal_spare(h, 0)) return set_error(GR_ENOMEM, "gr_batch: cannot allocate tuning spares");
   int rc = sync_problems(b);
   if (rc) return rc;
-  const int zcands[] = {0, 256, 128, 64};
+  // 32-plane items share out grids of up to 320 cells a side better (8 problems of 96..320:
+  // 295 us per step against 320 on 64-plane items); 256 planes were never the fastest
+  const int zcands[] = {0, 128, 64, 32};
   double best = 1e30;  // ms per step
   int bv = b->variant, bz = b->zchunk;
   for (int v = 0; v < kNumVariants; ++v) {
@@ -918,9 +926,10 @@ extern "C" int gr_batch_autotune(gr_batch *b, int steps, int use_graph, int *var
   bool fuse = false;
   if ((rc = fused_ready(b, &fuse))) return rc;
   const int passes = std::max(1, steps / 2);
+  const int w2_zcands[] = {0, 256, 128, 64};  // a block reads 8 more planes than it writes
   for (int wv = 0; wv < kNumW2 && fuse; ++wv) {
     if (b->w2_occupancy[wv] < 1 || (use_graph == 2 && b->w2_run_occupancy[wv] < 1)) continue;
-    for (int zc : zcands) {
+    for (int zc : w2_zcands) {
       b->w2_variant = wv;
       b->w2_zchunk = zc;
       if ((rc = build_w2_tables(b))) return rc;
