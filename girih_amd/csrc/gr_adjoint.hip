@@ -320,7 +320,7 @@ extern "C" int gr_shot_forward(gr_shot *s, void *rec_dev) {
   if (!s || !rec_dev) return gr::set_error(GR_EINVAL, "gr_shot_forward: null argument");
   gr_handle *h = s->h;
   const Problem &P = gr_internal_problem(h);
-  const gr::LaunchCfg &lc = gr_internal_launch_cfg(h);
+  gr::LaunchCfg lc = gr_internal_launch_cfg(h);
   hipStream_t st = gr_internal_stream(h);
   const size_t fbytes = (size_t)P.field_elems * gr::elem_size(P.dtype);
   const size_t plane = (size_t)P.nx * P.ny * gr::elem_size(P.dtype);
@@ -335,6 +335,7 @@ extern "C" int gr_shot_forward(gr_shot *s, void *rec_dev) {
     void *out = first ? s->ck[2 * c0] : second ? s->ck[2 * c1 + 1] : cur == s->x[0] ? s->x[1] : s->x[0];
     long long sidx = -1;
     const void *sv = src_of(h, a, &sidx);
+    lc.down = a & 1;
     e = gr::sweep_fields(P, fbase(P, out), fbase(P, cur), sv, sidx, lc, st, out == prev ? nullptr : fbase(P, prev));
     if (e == hipSuccess) e = record_any(P, fbase(P, out), s->rec_k, (char *)rec_dev + (size_t)a * plane, st);
     if (first && second && e == hipSuccess)  // checkpoints after every step: the state belongs to two
@@ -388,7 +389,7 @@ extern "C" int gr_shot_adjoint(gr_shot *s, const void *res_dev, void *grad_dev) 
   if (!s->have_forward) return gr::set_error(GR_EINVAL, "gr_shot_adjoint: run gr_shot_forward first");
   gr_handle *h = s->h;
   const Problem &P = gr_internal_problem(h);
-  const gr::LaunchCfg &lc = gr_internal_launch_cfg(h);
+  gr::LaunchCfg lc = gr_internal_launch_cfg(h);
   hipStream_t st = gr_internal_stream(h);
   const size_t fbytes = (size_t)P.field_elems * gr::elem_size(P.dtype);
   const size_t plane = (size_t)P.nx * P.ny * gr::elem_size(P.dtype);
@@ -440,6 +441,7 @@ extern "C" int gr_shot_adjoint(gr_shot *s, const void *res_dev, void *grad_dev) 
       const int t = a - a0 + 2;
       long long sidx = -1;
       const void *sv = src_of(h, a, &sidx);
+      lc.down = a & 1;
       e = gr::sweep_fields(P, xf(t), xf(t - 1), sv, sidx, lc, st, xf(t - 2));
     }
     // nu_{a1+2} and nu_{a1+3} are zero after the last step, else the two lowest of the
@@ -450,6 +452,7 @@ extern "C" int gr_shot_adjoint(gr_shot *s, const void *res_dev, void *grad_dev) 
     }
     for (int a = a1 - 1; a >= a0 && e == hipSuccess; --a) {  // nu_{a+2} <- f(nu_{a+3}, nu_{a+4}) + roc2 * residual
       const int t = a - a0;
+      lc.down = a & 1;
       e = gr::sweep_fields(P, nuf(t), nuf(t + 1), nullptr, -1, lc, st, nuf(t + 2));
       if (e == hipSuccess) e = inject_any(P, nuf(t), s->rec_k, (const char *)res_dev + (size_t)a * plane, st);
     }

@@ -26,6 +26,7 @@ struct LaunchCfg {
   int t_block = 1;  // fused time steps per pass
   int variant = 0;  // sweep tile variant (0 = default tile)
   int xcd_order = 1;  // renumber workgroups per XCD
+  bool down = false;  // planes taken from the top of z down (sweeps of kernels 0 to 4, kernel-5 passes)
   int ftile = 0;      // output tile of the fused pass, where its depth has several (fused_tiles)
   // settings the caller has not made: sweeps go by sweep_cfg's rule, fused passes by gr_step's
   bool auto_variant = false, auto_zchunk = false, auto_order = false;

@@ -67,11 +67,20 @@ int set_errorf(int code, const char *fmt, ...) {
 
 size_t elem_size(int dtype) { return dtype == GR_F64 ? 8 : 4; }
 
-int streaming_sweep(const Problem &P) {
-  if (P.strm_mode >= 0) return P.strm_mode;
+// Bytes that a sweep of P streams: both fields and the coefficient arrays.
+static double sweep_bytes(const Problem &P) {
   const double cbytes = (P.flags & GR_COEF_BF16) ? 2.0 : (double)elem_size(P.dtype);
   const double words = 2.0 * elem_size(P.dtype) + cbytes * (P.ncoef + (P.roc2 ? 1 : 0));
-  return (double)P.field_elems * words > 512.0 * 1024 * 1024 ? 1 : 0;  // 2x the 256 MB Infinity Cache
+  return (double)P.field_elems * words;
+}
+
+int streaming_sweep(const Problem &P) {
+  if (P.strm_mode >= 0) return P.strm_mode;
+  // The 256 MB Infinity Cache.  Kernel-0 sweeps of 250..520 MB gain 3..17% from the hints
+  // (FP32 with roc2 at 320^2 x 341, 400 MB: 278 -> 317 GLUP/s; FP64 at 256^2 x 266: 148 ->
+  // 168), those of 200 MB lose 1..6% and FP32 with scalar roc2 21%; fused passes of kernel 1
+  // gain 1..5% from 250 MB on, those of kernel 5 do not care.
+  return sweep_bytes(P) > 256.0 * 1024 * 1024 ? 1 : 0;
 }
 
 // ------------------------------------------------------------------ tile variants
@@ -136,10 +145,40 @@ LaunchCfg sweep_cfg(int kid, const LaunchCfg &lc, int nx, int ny, int nz) {
   return c;
 }
 
+// Whether successive sweeps or passes over P run up and down z in turn (LaunchCfg::down), so
+// that each starts with the planes that the one before touched last, while the 256 MB
+// Infinity Cache still holds them.  Kernel-0 sweeps, GLUP/s one way / in turn: FP32 with
+// roc2 at 288^2 x 316 (300 MB) 251 / 269 and at 400^3 (1 GB) 315 / 320, FP64 at 500 x 330 x
+// 270 (1.4 GB) 162 / 168 and at 768^2 x 512 (9 GB) 166 / 167; the same at 12 GB and within
+// the cache.  Kernel-5 passes: FP64 at 192^2 x 200 (500 MB) 190 / 205 and at 320^3 (2.2 GB)
+// 205 / 209, FP32 at 192^2 x 200 306 / 327, but FP64 at 512^3 (9 GB) 241 / 235.  Kernel-1
+// passes, bound by their arithmetic, gained nothing.
+static bool z_turns(const Problem &P) {
+  const double mb = sweep_bytes(P) / (1024 * 1024);
+  return P.kernel == 5 ? mb < 4096 : streaming_sweep(P) && mb < 10240;
+}
+
+// The same sweep with its planes numbered from the top: plane k of the arguments is plane
+// zb + ze - 1 - k of the fields.  Kernels 0 to 4 add the planes below and above in pairs, and
+// so give the same bits either way; kernel 5 does not (its passes have an instantiation
+// for it, its sweeps run up only).
+template <typename T, typename C>
+static void turn(SweepArgs<T, C> &a) {
+  const long long top = (a.g.zb + a.g.ze - 1) * a.g.sz;
+  a.u += top;
+  a.v += top;
+  if (a.uold) a.uold += top;
+  if (a.roc2) a.roc2 += top;
+  if (a.coef) a.coef += top;
+  if (a.src_k >= 0) a.src_k = a.g.zb + a.g.ze - 1 - a.src_k;
+  a.g.sz = -a.g.sz;
+}
+
 // One sweep u <- f(v) with the handle's configuration.
 hipError_t sweep_fields(const Problem &P, void *u, const void *v, const void *src, long long src_idx,
                         const LaunchCfg &cfg, hipStream_t st, const void *uold) {
   const LaunchCfg lc = sweep_cfg(P.kernel, cfg, P.nx, P.ny, P.nz);
+  const bool down = lc.down && P.kernel != 5 && z_turns(P);
   const bool fast = (P.flags & GR_FAST) != 0;
   const bool rocs = (P.flags & GR_ROC2_SCALAR) != 0;
   const bool bf16 = (P.flags & GR_COEF_BF16) != 0;
@@ -166,6 +205,7 @@ hipError_t sweep_fields(const Problem &P, void *u, const void *v, const void *sr
     a.src = (const double *)src;
     a.src_k = src_idx < 0 ? -1 : (int)(src_idx / g.sz);
     a.src_off = src_idx < 0 ? 0 : (int)(src_idx % g.sz);
+    if (down) turn(a);
     return launch_sweep_f64(P.kernel, false, rocs, a, lc, st, streaming_sweep(P));
   }
   if (bf16) {
@@ -183,6 +223,7 @@ hipError_t sweep_fields(const Problem &P, void *u, const void *v, const void *sr
     a.src = (const float *)src;
     a.src_k = src_idx < 0 ? -1 : (int)(src_idx / g.sz);
     a.src_off = src_idx < 0 ? 0 : (int)(src_idx % g.sz);
+    if (down) turn(a);
     return launch_sweep_bf16(P.kernel, fast, rocs, a, lc, st, streaming_sweep(P));
   }
   SweepArgs<float, float> a{};
@@ -199,6 +240,7 @@ hipError_t sweep_fields(const Problem &P, void *u, const void *v, const void *sr
   a.src = (const float *)src;
   a.src_k = src_idx < 0 ? -1 : (int)(src_idx / g.sz);
   a.src_off = src_idx < 0 ? 0 : (int)(src_idx % g.sz);
+  if (down) turn(a);
   return launch_sweep_f32(P.kernel, fast, rocs, a, lc, st, streaming_sweep(P));
 }
 
@@ -647,7 +689,9 @@ static hipError_t single_app(gr_handle *h, long long app) {
   const void *srcp = has_src ? (const char *)h->src + (size_t)app * es : nullptr;
   const long long sidx = has_src ? h->src_idx : -1;
   const int w = h->parity, r = 1 - w;
-  hipError_t e = sweep_fields(h->P, ubase(h, w), ubase(h, r), srcp, sidx, h->lc, h->stream);
+  LaunchCfg lc = h->lc;
+  lc.down = w == 1;
+  hipError_t e = sweep_fields(h->P, ubase(h, w), ubase(h, r), srcp, sidx, lc, h->stream);
   h->parity ^= 1;
   return e;
 }
@@ -795,7 +839,8 @@ static int enqueue_first_order(gr_handle *h, int napply, int *nlaunch) {
     const bool has_src = h->src && app < h->nsrc;
     const void *srcp = has_src ? (const char *)h->src + (size_t)app * es : nullptr;
     const long long sidx = has_src ? h->src_idx : -1;
-    const LaunchCfg lc = ops[i] > 1 ? fused_cfg(h, ops[i]) : h->lc;
+    LaunchCfg lc = ops[i] > 1 ? fused_cfg(h, ops[i]) : h->lc;
+    lc.down = (i & 1) && P.kernel == 5 && z_turns(P);
     const void *in = field_base(h, h->fbuf[x]);
     hipError_t e;
     if (i == m - 1) {
@@ -1033,11 +1078,12 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
   float best_ms = 1e30f;
   std::vector<std::pair<float, LaunchCfg>> tried;  // sweep trials: time of `steps` sweeps
   // one untimed sweep, then n timed sweeps
-  auto time_sweeps = [&](const LaunchCfg &lc, int n, float *ms) -> int {
+  auto time_sweeps = [&](LaunchCfg lc, int n, float *ms) -> int {
     hipError_t e = sweep_fields(P, a, b, nullptr, -1, lc, h->stream);
     if (e != hipSuccess) return fail(GR_EHIP, "autotune launch: %s", hipGetErrorString(e));
     HIP_TRY(hipEventRecord(h->ev0, h->stream));
     for (int s = 0; s < n; ++s) {
+      lc.down = !(s & 1);  // as steps do
       e = (s & 1) ? sweep_fields(P, a, b, nullptr, -1, lc, h->stream) : sweep_fields(P, b, a, nullptr, -1, lc, h->stream);
       if (e != hipSuccess) return fail(GR_EHIP, "autotune launch: %s", hipGetErrorString(e));
     }
@@ -1120,9 +1166,10 @@ extern "C" int gr_autotune(gr_handle *h, int steps, gr_stats *best) {
     const int nd = tb_depths(P.kernel, P.dtype, depths, 8);
     std::vector<std::pair<float, LaunchCfg>> fused;
     // one untimed pass, then npass timed passes: ms per `steps` applications, comparable with the sweep trials
-    auto time_passes = [&](const LaunchCfg &lc, int npass, float *per_step) -> int {
+    auto time_passes = [&](LaunchCfg lc, int npass, float *per_step) -> int {
       const int tl = lc.t_block;
       auto pass = [&](int q) {
+        lc.down = (q & 1) && P.kernel == 5 && z_turns(P);
         if (P.kernel == 0) return tblock_pass(P, tl, ubase(h, 0), ubase(h, 1), a, b, nullptr, -1, lc, h->stream);
         return tblock_pass(P, tl, nullptr, q & 1 ? b : a, nullptr, q & 1 ? a : b, nullptr, -1, lc, h->stream);
       };
@@ -1258,6 +1305,13 @@ extern "C" int gr_sweep_dev(int kernel, int dtype, const int shape[3], int xb, i
     P.coef = (void *)coef;
   }
   P.roc2 = (void *)roc2;
+  // Rows of the caller's layout start anywhere in a cache line, and a non-temporal store
+  // then writes parts of lines: for a 64-cell tile 2 of 3 lines in FP32, 2 of 5 in FP64.
+  // us per sweep without / with the hints: kernel 0 FP32 at 291^2 x 288 (300 MB) 113 / 130
+  // and at 515^2 x 494 486 / 593, kernel 5 FP32 at 291^2 x 309 207 / 238 and FP64 at 291^2 x
+  // 257 325 / 337; kernel 0 FP64 at 355^2 x 312 (1 GB) 314 / 300, kernel 1 FP64 at 355^2 x 312
+  // 168 / 159.
+  P.strm_mode = dtype == GR_F64 && P.ncoef == 0 && sweep_bytes(P) > 512.0 * 1024 * 1024;
   // express the box through the generic geometry
   Geom g;
   g.sy = shape[0];

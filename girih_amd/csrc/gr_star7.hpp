@@ -65,6 +65,7 @@ struct S7Args {
   const T *src;  // level t adds src[t-1] at plane src_k, in-plane element src_off from the
                  // row start (src_k < 0: no source)
   int src_k, src_off;
+  bool down;  // read by the host only: the DN instantiation, its planes numbered from the top
 };
 
 // P adjacent elements at byte offset `off` of a uniform base.
@@ -124,7 +125,7 @@ struct Star7 {
 };
 
 template <typename T, typename C, int KID, int TL, int TX, int TY, int NT, int P, int PD, bool STRM,
-          bool GEN>
+          bool GEN, bool DN>
 __global__ __launch_bounds__(NT) void star7_tb_kernel(const S7Args<T, C> a) {
   using G = Star7<T, C, KID, TL, TX, TY, NT, P>;
   constexpr int W = G::W, H = G::H, WS = G::WS, NS = G::NS, NR = G::NR, NC = G::NC, UN = G::UN;
@@ -319,7 +320,8 @@ __global__ __launch_bounds__(NT) void star7_tb_kernel(const S7Args<T, C> a) {
               else
                 c[m] = w;
             }
-            out = c[0] * v0 + c[1] * xm + c[2] * xp + c[3] * ym[e] + c[4] * yp[e] + c[5] * zm + c[6] * zp;
+            out = c[0] * v0 + c[1] * xm + c[2] * xp + c[3] * ym[e] + c[4] * yp[e] + c[5] * (DN ? zp : zm) +
+                  c[6] * (DN ? zm : zp);
           }
           if (GEN && srcp && off[j] + e * (unsigned)sizeof(T) == (unsigned)a.src_off * (unsigned)sizeof(T))
             out = out + a.src[t - 1];

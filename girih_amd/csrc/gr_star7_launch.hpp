@@ -16,10 +16,29 @@ static hipError_t launch_s7(S7Args<T, C> a, hipStream_t st) {
   a.zchunk = (a.zchunk <= 0 || a.zchunk > a.nz) ? a.nz : a.zchunk;
   a.nzc = (a.nz + a.zchunk - 1) / a.zchunk;
   const dim3 grid(a.tiles_x * a.tiles_y * a.nzc);
-  if (a.src_k >= 0 || a.Z1)
-    hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, PD, STRM, true>), grid, dim3(NT), 0, st, a);
+  const bool gen = a.src_k >= 0 || a.Z1;
+  if constexpr (KID == 5) {
+    if (a.down) {  // plane k of the arguments is plane nz + 1 - k of the fields
+      const long long top = (a.nz + 1) * a.sz;
+      a.Y += top;
+      a.Z += top;
+      if (a.Z1) a.Z1 += top;
+      a.coef += top;
+      if (a.src_k >= 0) a.src_k = a.nz + 1 - a.src_k;
+      a.sz = -a.sz;
+      if (gen)
+        hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, PD, STRM, true, true>), grid, dim3(NT), 0, st,
+                           a);
+      else
+        hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, PD, STRM, false, true>), grid, dim3(NT), 0, st,
+                           a);
+      return hipGetLastError();
+    }
+  }
+  if (gen)
+    hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, PD, STRM, true, false>), grid, dim3(NT), 0, st, a);
   else
-    hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, PD, STRM, false>), grid, dim3(NT), 0, st, a);
+    hipLaunchKernelGGL((star7_tb_kernel<T, C, KID, TL, TX, TY, NT, P, PD, STRM, false, false>), grid, dim3(NT), 0, st, a);
   return hipGetLastError();
 }
 
@@ -42,6 +61,7 @@ static S7Args<T, C> s7_args(const Problem &P, const void *Y, void *Z1, void *Z, 
   a.nz = P.nz;
   a.xcd_order = lc.xcd_order;
   a.zchunk = lc.zchunk;
+  a.down = lc.down;
   a.src = (const T *)src;
   a.src_k = src_idx < 0 ? -1 : (int)(src_idx / a.sz);
   a.src_off = src_idx < 0 ? 0 : (int)(src_idx % a.sz) + P.xoff;

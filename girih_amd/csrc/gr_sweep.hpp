@@ -341,7 +341,8 @@ __device__ __forceinline__ void SweepTile<T, C, KID, BY, RY, FAST, ROCS, RING, N
   auto plane = [&](const T *base, int k) { return base + (long long)k * g.sz; };
   const int zlast = g.ze + R - 1;  // last plane any load may touch
   // plane accesses: buffer resources (BUF) or SGPR-base global loads
-  const unsigned pbytes = (unsigned)g.sz * (unsigned)sizeof(T);
+  const unsigned psize = (unsigned)(g.sz < 0 ? -g.sz : g.sz);  // elements per plane
+  const unsigned pbytes = psize * (unsigned)sizeof(T);
   auto pl = [&](const T *base, int k) {
     if constexpr (BUF)
       return plane_rsrc(base + (long long)k * g.sz, pbytes);
@@ -395,7 +396,7 @@ __device__ __forceinline__ void SweepTile<T, C, KID, BY, RY, FAST, ROCS, RING, N
   auto load_u0 = [&](int k, T (&u_)[RY], T (&r_)[RY]) {
     if constexpr (KID == 0) {
       const auto up = pl(a.uold ? a.uold : a.u, k);
-      const unsigned cbytes = (unsigned)g.sz * (unsigned)sizeof(C);
+      const unsigned cbytes = psize * (unsigned)sizeof(C);
 #pragma unroll
       for (int m = 0; m < RY; ++m) {
         u_[m] = ld_strm(up, off[m]);
