@@ -38,7 +38,12 @@ namespace gr {
 namespace {
 
 // One problem of one step parity.  All words are 4-byte multiples (read with
-// readfirstlane into scalar registers).
+// readfirstlane into scalar registers).  Steps of parity 1 take the problems in the other
+// order and their planes from the top down (sz < 0, the pointers at the top plane), so that
+// they start with what the step before touched last and the Infinity Cache still holds;
+// kernel 0 adds the planes below and above in pairs, and so gives the same bits.  Us per
+// step one way / in turn: 12 bf16 problems of 96..320 cells a side (1.3 GB) 464 / 444, 11 of
+// them (1 GB) 353 / 344, 10 with FP32 roc2 (1.2 GB) 379 / 366, 16 of 192..512 (10 GB) the same.
 struct BatchDesc {
   float *u;          // written: u^(n+1) (holds u^(n-1) on entry)
   const float *v;    // read: u^n
@@ -52,6 +57,7 @@ struct BatchDesc {
   int src_k, src_off;
   float c[5], csum;
   int pad;
+  const float *field;  // the written field from its first plane (receivers)
 };
 static_assert(sizeof(BatchDesc) % 8 == 0, "descriptor words");
 
@@ -71,23 +77,24 @@ struct RecDesc {
 static_assert(sizeof(RecDesc) % 8 == 0, "descriptor words");
 
 // Row `row` of all receivers' planes after call step `step`, from the fields the step
-// wrote (table d of that step's parity); lanes stride over x.
-__device__ __forceinline__ void record_row(const BatchDesc *__restrict__ d, const RecDesc *__restrict__ r, int nrec,
-                                           int row, int step, int lane, int nlanes) {
+// wrote (table d of that step's parity: `odd`); lanes stride over x.
+__device__ __forceinline__ void record_row(const BatchDesc *__restrict__ d, int nprob, bool odd,
+                                           const RecDesc *__restrict__ r, int nrec, int row, int step, int lane,
+                                           int nlanes) {
   int ri = 0;
   while (ri + 1 < nrec && r[ri + 1].row0 <= row) ++ri;
   const RecDesc R = r[ri];
   const int j = row - R.row0, a = R.a0 + step;
   if (j >= R.ny || a >= R.max_steps) return;
-  const float *u = d[R.prob].u + R.plane + (long long)(j + 4) * R.sy + 4;
+  const float *u = d[odd ? nprob - 1 - R.prob : R.prob].field + R.plane + (long long)(j + 4) * R.sy + 4;
   float *t = R.trace + ((long long)a * R.ny + j) * R.nx;
   for (int i = lane; i < R.nx; i += nlanes) t[i] = u[i];
 }
 
 // The receivers of one step (launches per step): one workgroup per row.
-__global__ __launch_bounds__(256) void batch_record_kernel(const BatchDesc *__restrict__ d,
+__global__ __launch_bounds__(256) void batch_record_kernel(const BatchDesc *__restrict__ d, int nprob, bool odd,
                                                            const RecDesc *__restrict__ r, int nrec, int step) {
-  record_row(d, r, nrec, blockIdx.x, step, threadIdx.x, blockDim.x);
+  record_row(d, nprob, odd, r, nrec, blockIdx.x, step, threadIdx.x, blockDim.x);
 }
 
 constexpr int kMaxBatch = 256;
@@ -198,7 +205,7 @@ __global__ __launch_bounds__(64 * BX * BY) void batch_run_kernel(const BatchDesc
     step_items<C, BX, BY, RY, RING, LATE>(d + (size_t)(s & 1) * nprob, nprob, nitems, ctr, per * s, s, lds, sclaim);
     grid.sync();
     for (int row = blockIdx.x; row < nrows; row += gridDim.x)
-      record_row(d + (size_t)(s & 1) * nprob, rec, nrec, row, s, lane, nlanes);
+      record_row(d + (size_t)(s & 1) * nprob, nprob, s & 1, rec, nrec, row, s, lane, nlanes);
   }
 }
 
@@ -416,6 +423,20 @@ int build_tables(gr_batch *b, bool spares, int npasses = 0) {
   const BatchVariant &V = kVariants[b->variant];
   b->hdesc.assign(4 * (size_t)n, BatchDesc{});
   int item = 0;
+  // problem oi's descriptor in the table of step parity q
+  auto place = [&](BatchDesc E, int table, int q, int oi) {
+    E.field = E.u;
+    if (q == 1) {
+      const long long top = (E.ze + 3) * E.sz;  // planes 4 .. ze - 1 reflected
+      E.u += top;
+      E.v += top;
+      E.roc2 = (const char *)E.roc2 + top * (b->bf16 ? 2 : 4);
+      if (E.src_k >= 0) E.src_k = E.ze + 3 - E.src_k;
+      E.sz = -E.sz;
+      oi = n - 1 - oi;
+    }
+    b->hdesc[(size_t)(table + q) * n + oi] = E;
+  };
   for (int oi = 0; oi < n; ++oi) {
     const int i = b->order[oi];
     gr_handle *h = b->probs[i];
@@ -453,7 +474,7 @@ int build_tables(gr_batch *b, bool spares, int npasses = 0) {
       E.nsrc = has_src ? (int)(nsrc - done) : 0;
       E.src_k = has_src ? (int)(sidx / D.sz) : -1;
       E.src_off = has_src ? (int)(sidx % D.sz) : 0;
-      b->hdesc[(size_t)q * n + oi] = E;
+      place(E, 0, q, oi);
       if (spares) {
         BatchDesc S = D;
         S.u = (float *)gr_internal_spare(h, q);
@@ -461,10 +482,12 @@ int build_tables(gr_batch *b, bool spares, int npasses = 0) {
         if (!S.u || !S.v) return set_error(GR_ENOMEM, "gr_batch: cannot allocate tuning spares");
         S.src = nullptr;
         S.src_k = -1;
-        b->hdesc[(size_t)(2 + q) * n + oi] = S;
+        place(S, 2, q, oi);
       }
     }
   }
+  for (BatchDesc &E : b->hdesc)  // the other order counts the items from the other end
+    if (E.sz < 0) E.item0 = item - E.item0 - E.tiles_x * E.tiles_y * E.nzc;
   b->hrec.clear();
   b->nrows = 0;
   for (int oi = 0; oi < n && !spares; ++oi) {  // receivers of the problems (tuning records nothing)
@@ -587,7 +610,7 @@ hipError_t enqueue_steps(gr_batch *b, int table, int napply, int tblock, bool tu
     const BatchDesc *tab = b->ddesc + (size_t)(table + (q & 1)) * n;
     hipLaunchKernelGGL(f, dim3(b->grid), dim3(64 * V.bx, V.by), 0, st, tab, n, b->nitems, b->ctr, base, s);
     base += (unsigned long long)(b->nitems + b->grid);
-    if (nrec) hipLaunchKernelGGL(batch_record_kernel, dim3(b->nrows), dim3(256), 0, st, tab, b->drec, nrec, s);
+    if (nrec) hipLaunchKernelGGL(batch_record_kernel, dim3(b->nrows), dim3(256), 0, st, tab, n, (q & 1) != 0, b->drec, nrec, s);
   }
   return hipGetLastError();
 }
