@@ -22,6 +22,14 @@ namespace gr {
 //     832 lanes x 2 636; before 388.  Depth 6, 64 x 16, 1024 lanes x 2: 703; before 322
 //   FP64 depth 4: 64 x 8, 512 lanes x 2 cells 245 (6.6 TB/s); 1024 lanes x 1 187
 //     (spills), 32 x 18 210; before 128
+//   The tiles that 64 does not divide fill their lanes (56 + 8 margin cells are 16 slots
+//   of 4) and compute fewer margin cells per cell of output, and grids that 64-wide tiles
+//   overhang have another width to choose.  One call of 24 steps, GLUP/s, 64-wide tile /
+//   the other, FP32 64 x 16 / 56 x 22 / 48 x 26: 389 x 270 x 331 337 / 357 / 339, 448 x 330 x
+//   260 327 / 393 / 325, 130 x 410 x 90 248 / 310 / 312, 300 x 310 x 250 320 / 331 / 366, 512^3
+//   416 / 394 / 390; bf16 depth 6 64 x 16 / 52 x 22: 674 / 727, 600 x 130 x 333 463 / 624; FP64
+//   64 x 8 / 56 x 10: 448 x 330 x 260 182 / 199, 130 x 410 x 90 147 / 204, 512^3 212 / 176.
+//   Never the fastest: FP32 64 x 18, 32 x 38; bf16 56 x 38, 48 x 42, 40 x 28; FP64 40 x 14, 32 x 18.
 //   depth 2: FP32 64 x 32 245, 128 x 16 262 (before 217); bf16 64 x 32 382 (258);
 //     FP64 64 x 16 138 (104)
 template <typename T, typename C>
@@ -34,23 +42,34 @@ static hipError_t k5_dispatch(int tl, int tile, const S7Args<T, C> &a, hipStream
       if (tile == 2) return launch_s7<T, C, 5, 4, 64, 16, 832, 2, 1, false>(a, st);
       return launch_s7<T, C, 5, 4, 64, 32, 704, 4, 1, false>(a, st);
     }
-    if (tl == 6) return launch_s7<T, C, 5, 6, 64, 16, 1024, 2, 1, false>(a, st);
+    if (tl == 6) {
+      if (tile == 1) return launch_s7<T, C, 5, 6, 52, 22, 1024, 2, 1, false>(a, st);
+      return launch_s7<T, C, 5, 6, 64, 16, 1024, 2, 1, false>(a, st);
+    }
   } else if constexpr (sizeof(T) == 4) {
     if (tl == 2) {
       if (tile == 1) return launch_s7<T, C, 5, 2, 128, 16, 704, 4, 1, false>(a, st);
       return launch_s7<T, C, 5, 2, 64, 32, 640, 2, 1, false>(a, st);
     }
-    if (tl == 4) return launch_s7<T, C, 5, 4, 64, 16, 448, 4, 1, false>(a, st);
+    if (tl == 4) {
+      if (tile == 1) return launch_s7<T, C, 5, 4, 56, 22, 448, 4, 1, false>(a, st);
+      if (tile == 2) return launch_s7<T, C, 5, 4, 48, 26, 448, 4, 1, false>(a, st);
+      return launch_s7<T, C, 5, 4, 64, 16, 448, 4, 1, false>(a, st);
+    }
   } else {
     if (tl == 2) return launch_s7<T, C, 5, 2, 64, 16, 704, 2, 1, false>(a, st);
-    if (tl == 4) return launch_s7<T, C, 5, 4, 64, 8, 512, 2, 1, false>(a, st);
+    if (tl == 4) {
+      if (tile == 1) return launch_s7<T, C, 5, 4, 56, 10, 512, 2, 1, false>(a, st);
+      return launch_s7<T, C, 5, 4, 64, 8, 512, 2, 1, false>(a, st);
+    }
   }
   return hipErrorInvalidValue;
 }
 
 int k5_tiles(const Problem &P, int tl) {
-  if (P.flags & GR_COEF_BF16) return tl == 4 ? 3 : 1;
-  return P.dtype == GR_F32 && tl == 2 ? 2 : 1;
+  if (P.flags & GR_COEF_BF16) return tl == 4 ? 3 : tl == 6 ? 2 : 1;
+  if (P.dtype == GR_F64) return tl == 4 ? 2 : 1;
+  return tl == 2 ? 2 : tl == 4 ? 3 : 1;
 }
 
 template <typename T, typename C>
