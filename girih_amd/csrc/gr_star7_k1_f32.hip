@@ -13,14 +13,16 @@ namespace gr {
 // GLUP/s, against one-cell lanes (1029-1179 at depth 4); in parentheses with the input
 // loaded one plane ahead instead of two:
 //   depth 2: 128 x 32 1280 (1020), 128 x 16 1231 (1066);
-//   depth 3: 128 x 16 1624 (1478), 64 x 16 1352 (1113);
+//   depth 3: 128 x 16 1624 (1478);
 //   depth 4: 128 x 24 1714 three planes ahead, 1694 two (1472), 128 x 16 1690 (1279);
 //   depth 5: 128 x 16 1663 (1597; 1394 with 2 cells per lane);  depth 6: 64 x 20 1150 (1099).
 // The narrower tiles are for grids that 128-wide tiles would overhang: one call of 24 steps
 // at depth 4, 128 x 24 / 64 x 50 (1.26x the tile computed) / 48 x 26: 512^3 1539 / 1543 / 1365,
 // 448 x 330 x 260 1357 / 1625 / 1203, 389 x 270 x 331 1198 / 1366 / 1216, 130 x 410 x 90 577 /
-// 674 / 764, 192 x 180 x 230 873 / 1041 / 1059.  64 x 16 (1053, 584, 896 at the last three) and
-// 96 x 32 were never the fastest.
+// 674 / 764, 192 x 180 x 230 873 / 1041 / 1059.  600 x 130 x 333 1320 / 1319 / 1268 and 1459
+// on 56 x 26.  Depth 3, 128 x 16 / 64 x 24: 512^3 1449 / 1404, 251 x 420 x 140 1135 / 1368, 192 x
+// 180 x 230 754 / 1101.  Never the fastest: 64 x 16 at depths 3 and 4, 64 x 22 and 96 x 32 at 4,
+// 120 x 12 at 3, 56 x 44 at 5.
 template <bool STRM>
 static hipError_t k1_dispatch(int tl, int tile, const S7Args<float, float> &a, hipStream_t st) {
   switch (tl) {
@@ -28,12 +30,13 @@ static hipError_t k1_dispatch(int tl, int tile, const S7Args<float, float> &a, h
       if (tile == 1) return launch_s7<float, float, 1, 2, 128, 16, 704, 2, 2, STRM>(a, st);
       return launch_s7<float, float, 1, 2, 128, 32, 832, 2, 2, STRM>(a, st);
     case 3:
-      if (tile == 1) return launch_s7<float, float, 1, 3, 64, 16, 384, 2, 2, STRM>(a, st);
+      if (tile == 1) return launch_s7<float, float, 1, 3, 64, 24, 512, 4, 2, STRM>(a, st);
       return launch_s7<float, float, 1, 3, 128, 16, 704, 2, 2, STRM>(a, st);
     case 4:
       if (tile == 1) return launch_s7<float, float, 1, 4, 128, 24, 1024, 4, 3, STRM>(a, st);
       if (tile == 2) return launch_s7<float, float, 1, 4, 64, 50, 1024, 4, 3, STRM>(a, st);
       if (tile == 3) return launch_s7<float, float, 1, 4, 48, 26, 448, 4, 2, STRM>(a, st);
+      if (tile == 4) return launch_s7<float, float, 1, 4, 56, 26, 512, 4, 2, STRM>(a, st);
       return launch_s7<float, float, 1, 4, 128, 16, 768, 2, 2, STRM>(a, st);
     case 5: return launch_s7<float, float, 1, 5, 128, 16, 896, 4, 2, STRM>(a, st);
     case 6: return launch_s7<float, float, 1, 6, 64, 20, 640, 4, 2, STRM>(a, st);

@@ -316,7 +316,7 @@ int fused_tiles(const Problem &P, int tl) {
   if (P.kernel == 5) return k5_tiles(P, tl);
   if (P.kernel == 1) {
     if (P.dtype == GR_F64) return tl == 2 ? 2 : tl == 4 ? 3 : 1;
-    return tl == 2 || tl == 3 ? 2 : tl == 4 ? 4 : 1;
+    return tl == 2 || tl == 3 ? 2 : tl == 4 ? 5 : 1;
   }
   return 1;
 }
