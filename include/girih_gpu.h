@@ -135,7 +135,13 @@ int gr_sweep_dev(int kernel, int dtype, const int shape[3], int xb, int yb, int 
 
 /* Device pointer of a field for zero-copy interop: which = 0 U1, 1 U2, 2 roc2 / U3,
  * 3 coefficient arrays, 4 spare field A, 5 spare field B.  Layout via gr_get_stats:
- * element (i,j,k) at base + x_offset + (k*rows_y + j)*pitch_x + i. */
+ * element (i,j,k) at base + x_offset + (k*rows_y + j)*pitch_x + i.  The fields and spares
+ * trade buffers in fused steps, so ask again after a call that advances, uploads or
+ * initialises them.  The caller may rewrite a field through its pointer between calls
+ * (finished before the next one), boundary included: fused steps of a handle whose field
+ * pointers were handed out take the boundary from the fields anew at every call.  They
+ * need the same boundary in U1 and U2, which is checked after gr_upload and
+ * gr_init_fields only: rewrite both alike, or step with t_block 1. */
 int gr_field_ptr(gr_handle *h, int which, void **dev_ptr);
 
 /* Device-side initial states (no host traffic for large grids).
