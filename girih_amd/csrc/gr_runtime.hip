@@ -969,6 +969,14 @@ extern "C" int gr_run_ts(gr_handle *h, int ts, int nt, int t_dim, int *nt_applie
   return gr_step(h, ntr - 1);
 }
 
+// gr_set_config's and gr_stats' tile variant v + kTileBase * (t + 1) is the sweeps' variant v
+// with the passes' output tile t; below kTileBase the pass's tile goes by v, where the depth
+// has that many.
+constexpr int kTileBase = 64;
+static int default_ftile(const Problem &P, int depth, int variant) {
+  return variant < fused_tiles(P, depth) ? variant : 0;
+}
+
 extern "C" int gr_get_stats(gr_handle *h, gr_stats *out) {
   if (!h || !out) return fail(GR_EINVAL, "gr_get_stats: null argument");
   gr_stats s = h->stats;
@@ -988,7 +996,9 @@ extern "C" int gr_get_stats(gr_handle *h, gr_stats *out) {
   s.rows_y = h->P.rows;
   s.planes_z = h->P.planes;
   s.x_offset = h->P.xoff;
-  s.tile_variant = lc.variant;
+  s.tile_variant = lc.variant;  // one number that gr_set_config reads back to the same tiles
+  if (lc.t_block > 1 && lc.ftile != default_ftile(h->P, lc.t_block, lc.variant))
+    s.tile_variant += kTileBase * (lc.ftile + 1);
   s.xcd_order = lc.xcd_order;
   *out = s;
   return GR_OK;
@@ -996,16 +1006,23 @@ extern "C" int gr_get_stats(gr_handle *h, gr_stats *out) {
 
 extern "C" int gr_set_config(gr_handle *h, int variant, int zchunk, int t_block) {
   if (!h) return fail(GR_EINVAL, "gr_set_config: null handle");
+  const int depth = t_block >= 1 ? t_block : h->lc.t_block;
+  const int ftile = variant / kTileBase - 1;  // the pass's tile; -1: by the sweep's variant
+  if (variant >= kTileBase && (depth < 2 || ftile >= fused_tiles(h->P, depth)))
+    return fail(GR_EINVAL, "gr_set_config: pass tile %d not available for kernel %d at depth %d", ftile, h->P.kernel,
+                depth);
   if (variant >= 0) {
-    if (variant >= num_tile_variants(h->P.kernel, h->P.dtype))
-      return fail(GR_EINVAL, "gr_set_config: tile variant %d not available for kernel %d", variant, h->P.kernel);
-    h->lc.variant = variant;
+    if (variant % kTileBase >= num_tile_variants(h->P.kernel, h->P.dtype))
+      return fail(GR_EINVAL, "gr_set_config: tile variant %d not available for kernel %d", variant % kTileBase,
+                  h->P.kernel);
+    h->lc.variant = variant % kTileBase;
     h->lc.auto_variant = false;
   }
   if (zchunk >= 0) {
     h->lc.zchunk = zchunk;
     h->lc.auto_zchunk = false;
   }
+  const bool new_depth = t_block >= 1 && t_block != h->lc.t_block;
   if (t_block >= 1) {
     if (t_block > 1) {
       int depths[8];
@@ -1017,9 +1034,10 @@ extern "C" int gr_set_config(gr_handle *h, int variant, int zchunk, int t_block)
     }
     h->lc.t_block = t_block;
   }
-  // the fused pass's output tile goes by the tile variant where its depth has that many
-  if (variant >= 0 || t_block >= 1)
-    h->lc.ftile = h->lc.variant < fused_tiles(h->P, h->lc.t_block) ? h->lc.variant : 0;
+  if (variant >= kTileBase)
+    h->lc.ftile = ftile;
+  else if (variant >= 0 || new_depth)
+    h->lc.ftile = default_ftile(h->P, h->lc.t_block, h->lc.variant);
   return GR_OK;
 }
 

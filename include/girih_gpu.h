@@ -78,7 +78,7 @@ typedef struct gr_stats {
   int64_t device_bytes;      /* HBM held by the handle */
   int32_t pitch_x, rows_y, planes_z; /* device layout of one field */
   int32_t x_offset;          /* element offset of logical x = 0 within a row */
-  int32_t tile_variant;      /* gr_set_config tile variant in use */
+  int32_t tile_variant;      /* gr_set_config tile variant in use (64 and above: with a pass tile of its own) */
   int32_t xcd_order;         /* workgroup order (gr_set_xcd_order): 0 plain, 1 or 2 XCD-contiguous */
 } gr_stats;
 
@@ -156,7 +156,9 @@ int gr_init_coef_uniform(gr_handle *h, uint64_t seed, double lo0, double hi0, do
 
 /* Launch configuration: tile variant of the sweep kernel (0 = default; see
  * gr_get_stats for the resulting tile; where a fused depth has several output tiles,
- * variants 1, 2, .. below their number select those too), z planes streamed per workgroup (0 = all),
+ * variants 1, 2, .. below their number select those too, and v + 64 * (t + 1) selects
+ * variant v with the passes' tile t; gr_get_stats reports the form that selects what is
+ * in use, so its tile_variant, zchunk, t_block and xcd_order reproduce a tuning), z planes streamed per workgroup (0 = all),
  * fused time steps per HBM pass (1 = single sweep; kernel 0: 2; kernel 1: 2..6;
  * kernel 5: 2, 4, 6; other depths return GR_EUNSUPPORTED).  Fused passes run only
  * while U1 and U2 hold the same halo (with GR_COEF_BF16: kernels 0 and 5);
