@@ -289,6 +289,7 @@ struct gr_handle {
   hipGraphExec_t gexec = nullptr;
   GraphKey gkey{};
   int gparity = 0, glu[2] = {0, 1}, glaunches = 0;
+  int captures = 0;  // sequences captured so far
 };
 
 static void drop_graph(gr_handle *h);
@@ -675,6 +676,7 @@ static int ensure_spares(gr_handle *h, int n = 2);
 static int sync_spares(gr_handle *h);
 static int enqueue_apps(gr_handle *h, int napply, bool fuse, int *nlaunch);
 static int finish_step(gr_handle *h, int napply, int launches);
+static bool trades_buffers(const gr_handle *h, int napply);
 static void drop_graph(gr_handle *h) {
   if (h->gexec) {
     (void)hipStreamSynchronize(h->stream);  // a replay may still be running
@@ -737,7 +739,7 @@ extern "C" int gr_step(gr_handle *h, int napply) {
   GraphKey key{napply, h->parity, h->lu[0], h->lu[1], h->lc.variant, h->lc.zchunk, h->lc.t_block, h->lc.xcd_order,
                h->lc.ftile, h->lc.auto_variant + 2 * h->lc.auto_zchunk + 4 * h->lc.auto_order, fuse ? 1 : 0, -1};
   if (h->src && h->napplied < h->nsrc) key.napplied = h->napplied;  // source pointers are baked in
-  if (h->use_graph && napply > 0) {
+  if (h->use_graph && napply > 0 && !(fuse && trades_buffers(h, napply))) {
     if (!(h->gexec && h->gkey == key)) {
       drop_graph(h);
       const int parity0 = h->parity, lu0 = h->lu[0], lu1 = h->lu[1];
@@ -764,6 +766,7 @@ extern "C" int gr_step(gr_handle *h, int napply) {
         return fail(GR_EHIP, "step graph capture: %s", hipGetErrorString(e));
       }
       h->gkey = key;
+      ++h->captures;
     }
     HIP_TRY(hipEventRecord(h->ev0, h->stream));
     HIP_TRY(hipGraphLaunch(h->gexec, h->stream));
@@ -803,6 +806,27 @@ static LaunchCfg fused_cfg(const gr_handle *h, int tl) {
   return lc;
 }
 
+// Depth of the next launch of a first-order call with `rest` applications to go (1: a single sweep).
+static int rest_depth(const gr_handle *h, int rest) {
+  int depths[8], d = 1;
+  const int nd = tb_depths(h->P.kernel, h->P.dtype, depths, 8);
+  for (int i = 0; i < nd; ++i)
+    if (depths[i] <= std::min(rest, h->lc.t_block)) d = std::max(d, depths[i]);
+  return d;
+}
+
+// Whether a fused first-order call ends on other buffers than it began with
+// (enqueue_first_order): one pass, or one pass and an odd step's sweep.  Its one or two
+// launches are not captured: the sequence would differ at every call (128^3 FP64, 4 steps at
+// depth 4: 48 us, captured anew each time 61).
+static bool trades_buffers(const gr_handle *h, int napply) {
+  int sp[2];
+  spare_ids(h, sp);
+  if (h->P.kernel == 0 || napply < 2 || !h->fbuf[sp[0]]) return false;
+  const int d = rest_depth(h, napply);
+  return d == napply || (d == napply - 1 && (napply & 1));
+}
+
 // Launch napply applications of a first-order kernel as fused passes, the last of which
 // writes the field's last two levels (the U1/U2 pair a call leaves) into different
 // buffers, so that no single sweep is needed to make both exact: at 512^3, 20 kernel-5
@@ -811,19 +835,12 @@ static LaunchCfg fused_cfg(const gr_handle *h, int tl) {
 // application is left.  Three buffers take part: U1, U2 and a spare.  A pass may write
 // any buffer but the one it reads, so the sequence is led such that the call ends on
 // the buffers it began with (a captured graph then stays valid); only a call of one
-// pass has to trade the read field for the spare.
+// pass has to trade the read field for the spare (trades_buffers).
 static int enqueue_first_order(gr_handle *h, int napply, int *nlaunch) {
   const Problem &P = h->P;
   const size_t es = elem_size(P.dtype);
-  int depths[8];
-  const int nd = tb_depths(P.kernel, P.dtype, depths, 8);
   std::vector<int> ops;  // depth of each launch (1: a single sweep)
-  for (int rest = napply; rest > 0; rest -= ops.back()) {
-    int d = 1;
-    for (int i = 0; i < nd; ++i)
-      if (depths[i] <= std::min(rest, h->lc.t_block)) d = std::max(d, depths[i]);
-    ops.push_back(d);
-  }
+  for (int rest = napply; rest > 0; rest -= ops.back()) ops.push_back(rest_depth(h, rest));
   int sp[2];
   spare_ids(h, sp);
   const int m = (int)ops.size(), w = h->parity, r = 1 - w;
@@ -1787,6 +1804,7 @@ const void *gr_internal_source(const gr_handle *h, int *n, long long *idx) {
 }
 hipStream_t gr_internal_stream(const gr_handle *h) { return h->stream; }
 const gr::LaunchCfg &gr_internal_launch_cfg(const gr_handle *h) { return h->lc; }
+extern "C" int gr_internal_graph_captures(const gr_handle *h) { return h->captures; }
 int gr_internal_fused_prepare(gr_handle *h, bool *ok) {
   *ok = false;
   bool depth_ok = false;

@@ -179,7 +179,8 @@ int gr_set_streaming(gr_handle *h, int mode);
 /* Graph mode (no counterpart in girih): gr_step captures its launch sequence into a
  * HIP graph once and replays it while the step count, parity, configuration and
  * source window repeat (one launch per call instead of one per sweep; for small,
- * launch-bound grids).  Results are identical to eager launches. */
+ * launch-bound grids).  Calls of kernels 1 and 5 that are one fused pass (or one and an
+ * odd step's sweep) are launched directly.  Results are identical to eager launches. */
 int gr_set_graph(gr_handle *h, int on);
 /* Autotuner (replaces girih's CPU tile/thread-group search, diamond_utils.c:691-847):
  * times every tile variant x workgroup order x z-chunk x fused depth candidate for
