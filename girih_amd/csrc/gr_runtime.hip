@@ -267,6 +267,7 @@ struct gr_handle {
   void *fbuf[4] = {nullptr, nullptr, nullptr, nullptr};
   int lu[2] = {0, 1};
   bool spares_synced = false;  // spares hold the same halo as U1/U2
+  bool no_spare = false;       // no memory for a third buffer: not asked for again until the fields are set
   int halo_equal = -1;         // U1 and U2 hold the same halo (-1: not yet checked)
   bool exposed = false;        // gr_field_ptr gave a field's pointer away: the caller may write halos between calls
   void *alloc_roc2 = nullptr, *alloc_coef = nullptr;
@@ -310,6 +311,7 @@ static void state_reset(gr_handle *h) {
   h->parity = 0;
   h->napplied = 0;
   h->spares_synced = false;
+  h->no_spare = false;
   h->halo_equal = -1;
 }
 
@@ -726,13 +728,14 @@ extern "C" int gr_step(gr_handle *h, int napply) {
   const bool wave = h->P.kernel == 0;
   if (fuse && wave) {
     if ((rc = ensure_spares(h)) || (rc = sync_spares(h))) return rc;
-  } else if (fuse) {
+  } else if (fuse && !h->no_spare) {
     // a third buffer lets the last pass write both levels that a call leaves; without the
     // memory for it a call ends with a single sweep
     if (ensure_spares(h, 1) == GR_OK) {
       if ((rc = sync_spares(h))) return rc;
     } else {
       (void)hipGetLastError();
+      h->no_spare = true;
     }
   }
   // graph mode: replay the launch sequence of an identical earlier call
@@ -1079,8 +1082,11 @@ static int ensure_spares(gr_handle *h, int n) {
   const size_t fbytes = (size_t)h->P.field_elems * elem_size(h->P.dtype);
   for (int i = 2; i < 2 + n; ++i)
     if (!h->fbuf[i]) {
-      drop_graph(h);
-      HIP_TRY(hipMalloc(&h->fbuf[i], fbytes));
+      void *p = nullptr;
+      HIP_TRY(hipMalloc(&p, fbytes));
+      drop_graph(h);  // a captured sequence runs without it
+      h->fbuf[i] = p;
+      h->no_spare = false;
       HIP_TRY(hipMemsetAsync(h->fbuf[i], 0, fbytes, h->stream));  // ordered before the spares' first use
       h->spares_synced = false;
       h->stats.device_bytes += (int64_t)fbytes;
