@@ -501,6 +501,25 @@ static bool ensure_stage(gr_handle *h) {
   return ok;
 }
 
+// Makes a device current for a scope; the caller's own is current again after it.
+class CurrentDevice {
+ public:
+  explicit CurrentDevice(int device) {
+    int now = 0;
+    status = hipGetDevice(&now);
+    if (status == hipSuccess && now != device && (status = hipSetDevice(device)) == hipSuccess) back_ = now;
+  }
+  ~CurrentDevice() {
+    if (back_ >= 0) (void)hipSetDevice(back_);
+  }
+  CurrentDevice(const CurrentDevice &) = delete;
+  CurrentDevice &operator=(const CurrentDevice &) = delete;
+  hipError_t status;
+
+ private:
+  int back_ = -1;
+};
+
 // Host threads this process may use.
 static int host_threads() {
   cpu_set_t set;
@@ -515,7 +534,7 @@ static int copy_rows(gr_handle *h, char *dev, size_t dev_pitch, char *host, size
   std::atomic<int> next{0}, err{(int)hipSuccess};
   auto work = [&](int t) {
     char *slot = (char *)h->stage + (size_t)t * kStageBytes;
-    hipError_t e = hipSetDevice(h->device);
+    hipError_t e = t > 0 ? hipSetDevice(h->device) : hipSuccess;  // current on the caller's thread already
     bool busy = false;  // the slot is still being read by the unpacking kernel
     for (int c; e == hipSuccess && err.load() == (int)hipSuccess && (c = next.fetch_add(1)) < nchunk;) {
       const int r0 = c * per, n = std::min(per, nrows - r0);
@@ -556,6 +575,9 @@ static int copy_field(gr_handle *h, const int ld[3], void *dev_base, size_t dev_
   const size_t dpitch = (size_t)P.pitch * dev_es, hpitch = (size_t)ld[0] * host_es;
   const size_t nrows = (size_t)P.rows * P.planes;
   if (dev_es != host_es) return fail(GR_EINVAL, "copy_field: element size mismatch");
+  // slots, events and kernels belong to the handle's GPU, whichever is current
+  const CurrentDevice current(h->device);
+  if (current.status != hipSuccess) return fail(GR_EHIP, "copy_field: %s", hipGetErrorString(current.status));
   // memory that host threads cannot touch (a device pointer), and rows longer than a slot go to the runtime's copy
   hipPointerAttribute_t at{};
   const bool dev_mem = hipPointerGetAttributes(&at, host) == hipSuccess && at.type == hipMemoryTypeDevice;
