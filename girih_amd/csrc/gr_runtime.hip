@@ -284,6 +284,7 @@ struct gr_handle {
   int ncu = 1;         // compute units of the device
   // pinned slots of the host-field copies (copy_rows), one event each
   void *stage = nullptr;
+  size_t stage_bytes = 0;
   hipEvent_t stage_ev[8] = {};
   // graph mode (gr_set_graph): the last captured step sequence and the state it leaves
   bool use_graph = false;
@@ -453,7 +454,7 @@ __global__ void to_bf16_kernel(const float *src, __hip_bfloat16 *dst, long long 
 // them from it) over the bus while the other threads copy theirs between slot and
 // array, which also spreads the page faults of fresh arrays.
 constexpr int kStageThreads = 8;                  // host threads and slots
-constexpr size_t kStageBytes = (size_t)2 << 20;   // one slot
+constexpr size_t kStageBytes = (size_t)2 << 20;   // one slot (a copy that is smaller takes what it needs)
 
 // rows of `width` words at `pitch` <-> rows at `width` (one wavefront per row)
 template <typename W, bool PACK>
@@ -485,16 +486,22 @@ static void free_stage(gr_handle *h) {
   }
   if (h->stage) (void)hipHostFree(h->stage);
   h->stage = nullptr;
+  h->stage_bytes = 0;
 }
 
-// The handle's pinned slots, allocated on first use (false: not available).
-static bool ensure_stage(gr_handle *h) {
-  if (h->stage) return true;
-  bool ok = hipHostMalloc(&h->stage, kStageThreads * kStageBytes, hipHostMallocDefault) == hipSuccess;
+// At least `bytes` of pinned slots, kept until the handle is destroyed or a copy needs more
+// (false: not available).  A handle holds what its largest copy uses, at most 16 MB: one of 30^3
+// 128 KB.
+static bool ensure_stage(gr_handle *h, size_t bytes) {
+  if (h->stage_bytes >= bytes) return true;
+  free_stage(h);
+  bool ok = hipHostMalloc(&h->stage, bytes, hipHostMallocDefault) == hipSuccess;
   if (!ok) h->stage = nullptr;
   for (int i = 0; i < kStageThreads && ok; ++i)
     ok = hipEventCreateWithFlags(&h->stage_ev[i], hipEventDisableTiming) == hipSuccess;
-  if (!ok) {
+  if (ok) {
+    h->stage_bytes = bytes;
+  } else {
     (void)hipGetLastError();
     free_stage(h);
   }
@@ -527,13 +534,18 @@ static int host_threads() {
   return sched_getaffinity(0, sizeof(set), &set) == 0 ? std::max(1, CPU_COUNT(&set)) : 1;
 }
 
+// Copies nrows rows through the slots; *done false where there is no memory for them.
 static int copy_rows(gr_handle *h, char *dev, size_t dev_pitch, char *host, size_t host_pitch, size_t width, int nrows,
-                     size_t es, bool to_dev) {
-  const int per = (int)std::max<size_t>(1, kStageBytes / width);  // rows per chunk
+                     size_t es, bool to_dev, bool *done) {
+  const int per = (int)std::max<size_t>(1, std::min<size_t>(nrows, kStageBytes / width));  // rows per chunk
   const int nchunk = (nrows + per - 1) / per;
+  const int nt = std::min({kStageThreads, nchunk, host_threads()});
+  const size_t slot_bytes = (per * width + 63) / 64 * 64;
+  *done = ensure_stage(h, nt * slot_bytes);
+  if (!*done) return GR_OK;
   std::atomic<int> next{0}, err{(int)hipSuccess};
   auto work = [&](int t) {
-    char *slot = (char *)h->stage + (size_t)t * kStageBytes;
+    char *slot = (char *)h->stage + (size_t)t * slot_bytes;
     hipError_t e = t > 0 ? hipSetDevice(h->device) : hipSuccess;  // current on the caller's thread already
     bool busy = false;  // the slot is still being read by the unpacking kernel
     for (int c; e == hipSuccess && err.load() == (int)hipSuccess && (c = next.fetch_add(1)) < nchunk;) {
@@ -555,7 +567,6 @@ static int copy_rows(gr_handle *h, char *dev, size_t dev_pitch, char *host, size
     if (busy) (void)hipEventSynchronize(h->stage_ev[t]);
     if (e != hipSuccess) err.store((int)e);
   };
-  const int nt = std::min({kStageThreads, nchunk, host_threads()});
   std::vector<std::thread> pool;
   try {
     for (int t = 1; t < nt; ++t) pool.emplace_back(work, t);
@@ -585,9 +596,12 @@ static int copy_field(gr_handle *h, const int ld[3], void *dev_base, size_t dev_
   const bool direct = hipPointerGetAttributes(&at, host) == hipSuccess &&
                       (at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeHost);
   (void)hipGetLastError();
-  if (!direct && width <= kStageBytes && nrows <= (size_t)INT_MAX && ensure_stage(h))
-    return copy_rows(h, (char *)dev_base, dpitch, (char *)const_cast<void *>(host), hpitch, width, (int)nrows, dev_es,
-                     to_dev);
+  if (!direct && width <= kStageBytes && nrows <= (size_t)INT_MAX) {
+    bool done = false;
+    const int rc = copy_rows(h, (char *)dev_base, dpitch, (char *)const_cast<void *>(host), hpitch, width, (int)nrows,
+                             dev_es, to_dev, &done);
+    if (done) return rc;
+  }
   if (to_dev)
     HIP_TRY(hipMemcpy2DAsync(dev_base, dpitch, host, hpitch, width, nrows, hipMemcpyHostToDevice, h->stream));
   else
@@ -1836,7 +1850,7 @@ const void *gr_internal_source(const gr_handle *h, int *n, long long *idx) {
 hipStream_t gr_internal_stream(const gr_handle *h) { return h->stream; }
 const gr::LaunchCfg &gr_internal_launch_cfg(const gr_handle *h) { return h->lc; }
 extern "C" int gr_internal_graph_captures(const gr_handle *h) { return h->captures; }
-extern "C" long long gr_internal_pinned_bytes(const gr_handle *h) { return h->stage ? kStageThreads * kStageBytes : 0; }
+extern "C" long long gr_internal_pinned_bytes(const gr_handle *h) { return (long long)h->stage_bytes; }
 int gr_internal_fused_prepare(gr_handle *h, bool *ok) {
   *ok = false;
   bool depth_ok = false;

@@ -97,7 +97,9 @@ const char *gr_last_error(void);
  * arrays (coef[m*nnx*nny*nnz + idx], stencils.h:32) for kernels 2-5.  Any pointer
  * the kernel does not use may be NULL.  Element type follows desc.dtype; with
  * GR_COEF_BF16, U3 and coef are FP32 host arrays rounded to bf16 (nearest even) on
- * the device.  Resets the step parity (the next application writes U1). */
+ * the device.  Resets the step parity (the next application writes U1).  Pageable arrays
+ * pass through pinned host memory that the handle keeps until gr_destroy: the size of the
+ * largest array it has moved, at most 16 MB (gr_download and gr_download_roc2 too). */
 int gr_upload(gr_handle *h, const int ldomain_shape[3], const void *U1, const void *U2,
               const void *U3, const void *coef);
 /* Copy U1 and U2 back into girih-layout host arrays (either may be NULL). */

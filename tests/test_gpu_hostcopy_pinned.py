@@ -38,3 +38,20 @@ def test_arrays_arrive_whole(dtype, nx, ny, nz, pad, pinned):
     for u, d in ((U1, D1), (U2, D2)):
         np.testing.assert_array_equal(d[:, :, :nx + 2], u[:, :, :nx + 2])
         assert (d[:, :, nx + 2:] == 7).all()
+
+
+def test_slots_are_no_larger_than_the_copies():
+    dt = np.float32
+    for n, at_most in (((1, 1, 1), 4096), ((30, 30, 30), 1 << 18), ((254, 254, 126), 16 << 20)):
+        U = np.random.default_rng(n[0]).random((n[2] + 2, n[1] + 2, n[0] + 2)).astype(dt)
+        small = np.zeros((3, 3, 3), dt)
+        with gpu.Stepper(1, *n, dtype=gpu.GR_F32, coef=[0.4, 0.1]) as st, \
+                gpu.Stepper(1, 1, 1, 1, dtype=gpu.GR_F32, coef=[0.4, 0.1]) as other:
+            other.upload(small, small)
+            for _ in range(2):
+                st.upload(U, U)
+                D1, D2 = st.download(U.shape)
+                np.testing.assert_array_equal(D1, U)
+                np.testing.assert_array_equal(D2, U)
+            assert 0 < pinned_bytes(st) <= min(at_most, U.nbytes + 4096)
+            assert pinned_bytes(other) <= 4096
