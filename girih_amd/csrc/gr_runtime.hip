@@ -366,10 +366,10 @@ extern "C" int gr_create(const gr_desc *d, gr_handle **out) {
   P.field_elems = (long long)P.pitch * P.rows * P.planes;
   h->lc.zchunk = 0;
   h->lc.auto_variant = h->lc.auto_zchunk = true;
-  {  // GIRIH_XCD_ORDER=1 or 2 starts from that workgroup order (the autotuner tries all three)
+  {  // GIRIH_XCD_ORDER=0, 1 or 2 starts from that workgroup order (the autotuner tries all three)
     const char *e = getenv("GIRIH_XCD_ORDER");
-    h->lc.xcd_order = (e && (e[0] == '1' || e[0] == '2')) ? e[0] - '0' : 0;
-    h->lc.auto_order = h->lc.xcd_order == 0;
+    h->lc.auto_order = !(e && e[0] >= '0' && e[0] <= '2');
+    h->lc.xcd_order = h->lc.auto_order ? 0 : e[0] - '0';
   }
   h->lc.t_block = d->t_block <= 0 ? 1 : d->t_block;  // 0: single sweeps until gr_autotune picks a depth
   if (h->lc.t_block > 1) {
