@@ -22,7 +22,7 @@
 // states from its checkpoint, read in place, into a buffer and walks it backwards, the
 // adjoint fields of the segments following each other in a ring (400^3 FP32, 100 steps,
 // checkpoints every 50: 71.4 -> 70.1 ms without the fields' copies).  Memory: 2*ceil(nt/K) + 2 fields for the forward pass;
-// the first backward pass adds 2K + 4 fields (the segment's states and adjoint
+// the first backward pass adds 2K + 2 fields (K states of the segment, K + 2 adjoint
 // fields) and a dense accumulator, which takes a segment's gradient terms in one pass.
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
@@ -68,9 +68,9 @@ __global__ void inject_kernel_same(T *nu, const T *roc2, long long sy, long long
 // walk, as the CPU adjoint adds them, but g is read and written once per segment and
 // each state and adjoint field once.  The differences are formed in FP64 (exact for
 // FP32 states); g has the field type: an FP32 shot's gradient error is set by its FP32
-// traces, far above FP32 accumulation over the steps.  States x_{a0} .. x_{a1+1} are
-// fields xs + t * fstride; nu_{a+2} is field nus + (a - a0) * fstride.  The source
-// term applies at cell src_idx for steps a < nsrc.
+// traces, far above FP32 accumulation over the steps.  States x_{a0} and x_{a0+1} are
+// x0 and x1, x_{a0+2} .. x_{a1+1} the fields from xs on; nu_{a+2} is field nub + a - a0 of
+// the ring nus.  The source term applies at cell src_idx for steps a < nsrc.
 template <typename T>
 __global__ void grad_segment_kernel(T *g, const T *__restrict__ nus, int nub, int nring, const T *__restrict__ x0,
                                     const T *__restrict__ x1, const T *__restrict__ xs, long long fstride,
@@ -82,7 +82,7 @@ __global__ void grad_segment_kernel(T *g, const T *__restrict__ nus, int nub, in
   T &gc = g[((long long)k * ny + j) * nx + i];
   T acc = gc;
   const bool at_src = src && o == src_idx;
-  auto xf = [&](int t) { return t == 0 ? x0 : t == 1 ? x1 : xs + (long long)t * fstride; };
+  auto xf = [&](int t) { return t == 0 ? x0 : t == 1 ? x1 : xs + (long long)(t - 2) * fstride; };
   auto nuf = [&](int t) { return nus + (long long)(nub + t < nring ? nub + t : nub + t - nring) * fstride; };
   double xa2 = (double)xf(nsteps + 1)[o];  // x_{a+2} for a = a1 - 1
   double xa1 = (double)xf(nsteps)[o];
@@ -163,7 +163,7 @@ struct gr_shot {
   double dt_over_h = 0;
   std::vector<void *> allocs;  // everything below lives in these
   std::vector<void *> ck;      // 2*nck checkpoint fields (x_{cK}, x_{cK+1})
-  void *seg = nullptr;         // ckpt+2 recompute fields; x_{a0+t} in field t for t >= 2
+  void *seg = nullptr;         // ckpt recompute fields, x_{a0+2} .. x_{a1+1}
   void *nus = nullptr;         // ckpt+2 adjoint fields nu_{a0+2} .. nu_{a1+3}, a ring over the segments
   void *x[2] = {nullptr, nullptr};  // forward states between checkpoints
   void *g = nullptr;  // gradient accumulator, field type, dense interior
@@ -395,7 +395,7 @@ extern "C" int gr_shot_adjoint(gr_shot *s, const void *res_dev, void *grad_dev) 
   const size_t plane = (size_t)P.nx * P.ny * gr::elem_size(P.dtype);
   const long long ncell = (long long)P.nx * P.ny * P.nz;
   hipError_t e = hipSuccess;
-  const int nslot = s->ckpt + 2;
+  const int nring = s->ckpt + 2;
   if (!s->seg) {  // backward-pass buffers, allocated on first use (forward-only shots never hold them)
     const size_t before = s->allocs.size();
     auto fields = [&](void **p, int n) -> hipError_t {
@@ -404,8 +404,8 @@ extern "C" int gr_shot_adjoint(gr_shot *s, const void *res_dev, void *grad_dev) 
       if (r == hipSuccess) r = hipMemsetAsync(*p, 0, fbytes * (size_t)n, st);  // zero halo, ordered before first use
       return r;
     };
-    e = fields(&s->seg, nslot);
-    if (e == hipSuccess) e = fields(&s->nus, nslot);
+    e = fields(&s->seg, s->ckpt);
+    if (e == hipSuccess) e = fields(&s->nus, nring);
     if (e == hipSuccess) {
       e = hipMalloc(&s->g, gr::elem_size(P.dtype) * (size_t)ncell);
       if (e == hipSuccess) s->allocs.push_back(s->g);
@@ -418,7 +418,6 @@ extern "C" int gr_shot_adjoint(gr_shot *s, const void *res_dev, void *grad_dev) 
       return gr::set_errorf(GR_ENOMEM, "gr_shot_adjoint: device allocation failed: %s", hipGetErrorString(e));
     }
   }
-  const int nring = nslot;
   int nub = 0;  // ring field of the segment's nu_{a0+2}
   if (e == hipSuccess) {
     if (P.dtype == GR_F64)
@@ -432,7 +431,7 @@ extern "C" int gr_shot_adjoint(gr_shot *s, const void *res_dev, void *grad_dev) 
   for (int c = s->nck - 1; c >= 0 && e == hipSuccess; --c) {
     const int a0 = c * s->ckpt, a1 = std::min(a0 + s->ckpt, s->nt), K = a1 - a0;
     auto xf = [&](int t) {  // x_{a0+t}: the checkpoint, then the recomputed states
-      return fbase(P, t < 2 ? s->ck[2 * c + t] : (void *)((char *)s->seg + (size_t)t * fbytes));
+      return fbase(P, t < 2 ? s->ck[2 * c + t] : (void *)((char *)s->seg + (size_t)(t - 2) * fbytes));
     };
     auto nuf = [&](int t) {  // nu_{a0+2+t}
       return fbase(P, (char *)s->nus + (size_t)((nub + t) % nring) * fbytes);
