@@ -168,7 +168,8 @@ def main():
         st.autotune(4)
     s = st.stats()
     tb = s["t_block"]
-    # whole fused passes (first-order kernels end a step count with one single sweep)
+    # whole fused passes; first-order kernels take one step more, a single sweep, so that no
+    # pass is the kind that ends a call and writes a level more than the others
     napply = a.steps * tb + (0 if a.kernel == 0 or tb == 1 else 1)
     if a.warmup:
         st.step(tb if a.kernel == 0 or tb == 1 else tb + 1)  # loads the code objects
