@@ -40,7 +40,6 @@ template <typename T>
 struct TbArgs {
   const T *Y;   // level 0
   T *ZN;        // level TL
-  T *ZO;        // level TL-1 (null: not written)
   const T *coef;
   long long cstride;
   long long sy, sz;
@@ -235,12 +234,7 @@ __global__ __launch_bounds__(NT) void tb_kernel(const TbArgs<T> a) {
           for (int j = 0; j < NCOL; ++j)
             if (colv[j]) Lt[lofs[j]] = qv[t < TL ? t : 0][j][sl];
         }
-        // output: level TL into ZN (and level TL-1 into ZO) -- planes of the box
-        if (t == TL - 1 && a.ZO && live && zin && p >= zs && p < ze) {
-#pragma unroll
-          for (int j = 0; j < NCOL; ++j)
-            if (outc[j]) stb<T>(a.ZO + (long long)p * a.sz, off[j], val[j]);
-        }
+        // output: level TL into ZN -- planes of the box
         if (t == TL && live && zin && p >= zs && p < ze) {
 #pragma unroll
           for (int j = 0; j < NCOL; ++j)
@@ -288,13 +282,12 @@ int tb_depths(int kid, int dtype, int *out, int max) {
 }
 
 template <typename T>
-static hipError_t tb6_pass(const Problem &P, const void *Y, void *ZO, void *ZN, const void *src, long long src_idx,
+static hipError_t tb6_pass(const Problem &P, const void *Y, void *ZN, const void *src, long long src_idx,
                            const LaunchCfg &lc, hipStream_t st) {
   const long long sz = (long long)P.pitch * P.rows;
   TbArgs<T> a{};
   a.Y = (const T *)Y;
   a.ZN = (T *)ZN;
-  a.ZO = (T *)ZO;
   a.coef = (const T *)P.coef;
   a.cstride = P.field_elems;
   a.sy = P.pitch;
@@ -345,8 +338,9 @@ hipError_t tblock_pass(const Problem &P, int tl, const void *X, const void *Y, v
                              : k1_pass_f32(P, tl, Y, ZO, ZN, src, src_idx, lc, st);
   if (P.kernel != 5) return hipErrorInvalidValue;
   if (tl == 6 && !(P.flags & GR_COEF_BF16)) {
-    if (P.dtype == GR_F64) return tb6_pass<double>(P, Y, ZO, ZN, src, src_idx, lc, st);
-    return tb6_pass<float>(P, Y, ZO, ZN, src, src_idx, lc, st);
+    if (ZO) return hipErrorInvalidValue;  // the call's last pass is a shallower one
+    if (P.dtype == GR_F64) return tb6_pass<double>(P, Y, ZN, src, src_idx, lc, st);
+    return tb6_pass<float>(P, Y, ZN, src, src_idx, lc, st);
   }
   return k5_pass(P, tl, Y, ZO, ZN, src, src_idx, lc, st);
 }

@@ -18,7 +18,7 @@ def captures(st):
 # parity, and with it the sequence, from call to call: they are captured at every one.
 @pytest.mark.parametrize("kernel,dtype,depth,steps,most", [
     (1, gpu.GR_F64, 4, 4, 0), (1, gpu.GR_F32, 4, 2, 0), (1, gpu.GR_F32, 3, 3, 0), (1, gpu.GR_F64, 4, 5, 0),
-    (5, gpu.GR_F64, 4, 4, 0), (5, gpu.GR_F32, 6, 6, 0), (5, gpu.GR_F32, 2, 3, 0), (1, gpu.GR_F64, 4, 8, 1),
+    (5, gpu.GR_F64, 4, 4, 0), (5, gpu.GR_F32, 6, 6, 1), (5, gpu.GR_F32, 2, 3, 0), (1, gpu.GR_F64, 4, 8, 1),
     (1, gpu.GR_F32, 3, 4, 1), (5, gpu.GR_F32, 4, 20, 1), (1, gpu.GR_F64, 4, 7, 7)])
 def test_calls_capture_once_at_most(kernel, dtype, depth, steps, most):
     (eager, graph), shape = _pair(kernel, 70, 19, 13, dtype)
