@@ -342,18 +342,20 @@ struct BatchVariant {
 // (16 problems of 192..512 with bf16 roc2, 64-plane items, us per step with / without):
 // 64 x 32 2149 / 2398, its ring 1993 / 2042, 64 x 16 ring of 256 lanes 2064 / 2149, 128 x 16
 // ring of 1024 lanes 2106 / 2164; but 64 x 16 of 256 lanes 2830 / 2113, its ring of 512
-// lanes 2111 / 2072, 128 x 16 ring of 512 lanes 2299 / 2056.
-#define GR_BV(BX, BY, RY, RING, LATE)                                                        \
+// lanes 2111 / 2072, 128 x 16 ring of 512 lanes 2299 / 2056.  LRUN16 says it for the bf16 kernel
+// of whole calls: 64 x 32 (5 problems of 64..320, 12 steps, whole-z items) 5822 / 3609 us,
+// the others as LATE.
+#define GR_BV(BX, BY, RY, RING, LATE, LRUN16)                                                  \
   {                                                                                          \
     BX, BY, RY, RING, &batch_kernel<float, BX, BY, RY, RING, LATE>,                          \
         &batch_kernel<__hip_bfloat16, BX, BY, RY, RING, LATE>,                               \
         &batch_run_kernel<float, BX, BY, RY, RING, LATE>,                                    \
-        &batch_run_kernel<__hip_bfloat16, BX, BY, RY, RING, LATE>                            \
+        &batch_run_kernel<__hip_bfloat16, BX, BY, RY, RING, LRUN16>                          \
   }
-const BatchVariant kVariants[] = {GR_BV(1, 8, 4, false, true), GR_BV(1, 8, 4, true, true),
-                                  GR_BV(1, 4, 4, false, false), GR_BV(1, 8, 2, true, false),
-                                  GR_BV(1, 4, 4, true, true),  GR_BV(2, 8, 2, true, true),
-                                  GR_BV(2, 4, 4, true, false)};
+const BatchVariant kVariants[] = {GR_BV(1, 8, 4, false, true, false),  GR_BV(1, 8, 4, true, true, true),
+                                  GR_BV(1, 4, 4, false, false, false), GR_BV(1, 8, 2, true, false, false),
+                                  GR_BV(1, 4, 4, true, true, true),    GR_BV(2, 8, 2, true, true, true),
+                                  GR_BV(2, 4, 4, true, false, false)};
 #undef GR_BV
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
