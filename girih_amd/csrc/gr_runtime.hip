@@ -123,14 +123,20 @@ void tile_of_variant(int kid, int dtype, int variant, int *tx, int *ty) {
 //    1490 us, 8 1534, 16 1558; 403 x 300 x 219 kernel 4 384, 405, 419);
 //  * tile: 128 x 16 of 1024 lanes (for kernel 0 with the operand prefetch) where it overhangs
 //    the box no further than 64 x 16 does (256^3 kernel 0 FP32 60 us against 62, 512^3
-//    486 against 520; but 320^3 138 against 133) and there is work for 256 of them; else
-//    64 x 16 of 512 lanes (64^3 kernel 0 19 us against 22);
+//    486 against 520; but 320^3 138 against 133) and there is work for 256 of them, or with
+//    chunks of the caller's for 256 (kernel 0) or 150 (us per four sweeps, wide / 64 x 16: 152
+//    workgroups, 128 x 300 x 128 at 16 planes, kernel 0 FP32 102 / 97, kernel 1 FP64 73 / 79; 144, kernel 0
+//    FP64 384 x 384 x 100 at 64 planes 638 / 468; 64, kernel 5 FP64 250 x 120 x 200 936 / 583);
+//    else 64 x 16 of 512 lanes (64^3 kernel 0 19 us against 22);
 //  * order: XCD bands of tile rows (403 x 300 x 219 kernel 3 157 us, plain runs 164).
 LaunchCfg sweep_cfg(int kid, const LaunchCfg &lc, int nx, int ny, int nz) {
   LaunchCfg c = lc;
   const bool hot = kid == 0 || kid == 1 || kid == 5;  // kernels with tile variants
   if (lc.auto_variant) {
-    const bool wide = (nx + 127) / 128 * 2 == (nx + 63) / 64 && (long long)nx * ny * nz >= (1 << 21);
+    const long long chunks = lc.zchunk > 0 && lc.zchunk < nz ? (nz + lc.zchunk - 1) / lc.zchunk : 1;  // the caller's
+    const bool enough = lc.auto_zchunk ? (long long)nx * ny * nz >= (1 << 21)
+                                       : (nx + 127) / 128 * ((ny + 15) / 16) * chunks >= (kid == 0 ? 256 : 150);
+    const bool wide = (nx + 127) / 128 * 2 == (nx + 63) / 64 && enough;
     c.variant = !hot ? 0 : !wide ? 2 : kid == 0 ? 16 : 13;
   }
   if (lc.auto_zchunk) {
