@@ -84,9 +84,10 @@ long long gr_internal_napplied(const gr_handle *h);
 const void *gr_internal_source(const gr_handle *h, int *n, long long *idx);
 hipStream_t gr_internal_stream(const gr_handle *h);
 const gr::LaunchCfg &gr_internal_launch_cfg(const gr_handle *h);
-// Launch sequences that gr_step has captured for the handle, and the pinned host memory that
-// its copies hold (read by the tests).
+// Launch sequences that gr_step has captured for the handle, whether its sweeps use the cache
+// hints, and the pinned host memory that its copies hold (read by the tests).
 extern "C" int gr_internal_graph_captures(const gr_handle *h);
+extern "C" int gr_internal_streaming(const gr_handle *h);
 extern "C" long long gr_internal_pinned_bytes(const gr_handle *h);
 // One field of the problem's type between the device layout (x offset applied) and a host
 // array in girih's layout ld.  Complete when the handle's stream is.

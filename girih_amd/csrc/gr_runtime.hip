@@ -67,20 +67,35 @@ int set_errorf(int code, const char *fmt, ...) {
 
 size_t elem_size(int dtype) { return dtype == GR_F64 ? 8 : 4; }
 
-// Bytes that a sweep of P streams: both fields and the coefficient arrays.
-static double sweep_bytes(const Problem &P) {
+// Bytes per cell that a sweep of P streams: both fields and the coefficient arrays.
+static double cell_bytes(const Problem &P) {
   const double cbytes = (P.flags & GR_COEF_BF16) ? 2.0 : (double)elem_size(P.dtype);
-  const double words = 2.0 * elem_size(P.dtype) + cbytes * (P.ncoef + (P.roc2 ? 1 : 0));
-  return (double)P.field_elems * words;
+  return 2.0 * elem_size(P.dtype) + cbytes * (P.ncoef + (P.roc2 ? 1 : 0));
 }
+static double sweep_bytes(const Problem &P) { return (double)P.field_elems * cell_bytes(P); }
 
+// Whether sweeps and kernel-1 passes mark what they touch once as non-temporal: where the 256
+// MB Infinity Cache no longer holds it from one sweep to the next.  The fields with their rows'
+// padding must exceed it (kernel 1 FP64 384 x 384 x 100, 250 MB: 51 us a sweep without the hints,
+// 55 with), and their cells a line that differs by kernel, as sweeps of more arrays lose more
+// below it (kernel 5 FP32 128 x 300 x 128 has 175 MB of cells in 259 MB: 67 us without, 85 with).
+// us per sweep without / with, cubes and 128-wide boxes (MB of cells):
+//   kernel 0 FP64 225 67 / 72, 262 98 / 99, 301 121 / 119; FP32 201 60 / 64, 222 80 / 80, 294 95 / 90
+//   kernel 1 FP64 240 56 / 55, 278 71 / 66; FP32 184 47.5 / 44.9, 239 57 / 56, 274 69 / 64
+//   kernel 2 FP64 206 42 / 43, 240 51 / 50; FP32 186 43.9 / 42.6, 206 48.5 / 45.5
+//   kernel 3 FP64 309 61 / 63, 346 71 / 69; FP32 186 39.3 / 38.9, 206 44 / 42, 240 52 / 48
+//   kernel 4 FP64 332 61 / 66, 356 77 / 77, 393 74 / 73; FP32 312 64 / 65, 345 69 / 67
+//   kernel 5 FP64 289 64 / 70, 308 65 / 65, 346 72 / 70; FP32 288 53 / 56, 309 67 / 67, 342 71 / 67;
+//     bf16 206 43.3 / 43.1, 241 52 / 51, 309 65 / 63
+// Passes of kernel 1 gain 1..5% from 250 MB on, those of kernel 5 do not care.
 int streaming_sweep(const Problem &P) {
   if (P.strm_mode >= 0) return P.strm_mode;
-  // The 256 MB Infinity Cache.  Kernel-0 sweeps of 250..520 MB gain 3..17% from the hints
-  // (FP32 with roc2 at 320^2 x 341, 400 MB: 278 -> 317 GLUP/s; FP64 at 256^2 x 266: 148 ->
-  // 168), those of 200 MB lose 1..6% and FP32 with scalar roc2 21%; fused passes of kernel 1
-  // gain 1..5% from 250 MB on, those of kernel 5 do not care.
-  return sweep_bytes(P) > 256.0 * 1024 * 1024 ? 1 : 0;
+  static const int line_mb[6][3] = {{256, 225, 210}, {235, 180, 180}, {230, 180, 180},  // FP64, FP32, bf16 arrays
+                                    {330, 180, 180}, {340, 330, 300}, {310, 310, 235}};
+  constexpr double mb = 1024.0 * 1024.0;
+  const double cells = (double)(P.nx + 2 * P.R) * (P.ny + 2 * P.R) * (P.nz + 2 * P.R);
+  const int type = P.dtype == GR_F64 ? 0 : (P.flags & GR_COEF_BF16) ? 2 : 1;
+  return sweep_bytes(P) > 256 * mb && cells * cell_bytes(P) > line_mb[P.kernel][type] * mb ? 1 : 0;
 }
 
 // ------------------------------------------------------------------ tile variants
@@ -1860,6 +1875,7 @@ const void *gr_internal_source(const gr_handle *h, int *n, long long *idx) {
 hipStream_t gr_internal_stream(const gr_handle *h) { return h->stream; }
 const gr::LaunchCfg &gr_internal_launch_cfg(const gr_handle *h) { return h->lc; }
 extern "C" int gr_internal_graph_captures(const gr_handle *h) { return h->captures; }
+extern "C" int gr_internal_streaming(const gr_handle *h) { return streaming_sweep(h->P); }
 extern "C" long long gr_internal_pinned_bytes(const gr_handle *h) { return (long long)h->stage_bytes; }
 int gr_internal_fused_prepare(gr_handle *h, bool *ok) {
   *ok = false;

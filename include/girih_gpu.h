@@ -174,9 +174,10 @@ int gr_set_config(gr_handle *h, int tile_variant, int zchunk, int t_block);
 int gr_set_xcd_order(gr_handle *h, int xcd_order);
 /* Cache policy of the sweeps and fused passes (no counterpart in girih): mode -1
  * (default) uses non-temporal loads and stores for the data a step touches once when
- * the problem's working set exceeds 256 MB (the Infinity Cache), and normal
- * accesses otherwise; 0 never uses them; 1 always does.  The arithmetic is the same
- * in every mode: results never depend on it. */
+ * its fields and coefficients exceed the 256 MB Infinity Cache and their cells, without
+ * the rows' padding, 180 to 340 MB, by kernel and type; normal accesses otherwise; 0
+ * never uses them; 1 always does.  The arithmetic is the same in every mode: results
+ * never depend on it. */
 int gr_set_streaming(gr_handle *h, int mode);
 /* Graph mode (no counterpart in girih): gr_step captures its launch sequence into a
  * HIP graph once and replays it while the step count, parity, configuration and
