@@ -6,9 +6,9 @@
 
 namespace gr {
 
-// A pass is bound by the vector ALU (11 instructions per computed cell, 10 of them the
-// stencil; 86% busy at depth 5) and by the LDS reads behind each barrier, not by memory,
-// so a tile trades the margins it computes twice (1.33x the tile at 128 x 24, depth 4)
+// A pass is bound by the vector ALU (12.3 instructions per computed cell, 10 of them the
+// stencil; 77% busy on 64 x 50 at depth 4) and by the LDS reads behind each barrier, not by
+// memory (1.80 GB a pass at 512^3), so a tile trades the margins it computes twice (1.33x the tile at 128 x 24, depth 4)
 // against two workgroups per CU, which cover each other's barriers.  512^3, one box,
 // GLUP/s, against one-cell lanes (1029-1179 at depth 4); in parentheses with the input
 // loaded one plane ahead instead of two:
