@@ -28,6 +28,7 @@ struct LaunchCfg {
   int xcd_order = 1;  // renumber workgroups per XCD
   bool down = false;  // planes taken from the top of z down (sweeps of kernels 0 to 4, kernel-5 passes)
   int ftile = 0;      // output tile of the fused pass, where its depth has several (fused_tiles)
+  void *halo = nullptr;  // star7 passes: a field (x offset applied) that takes the input's halo on the way
   // settings the caller has not made: sweeps go by sweep_cfg's rule, fused passes by gr_step's
   bool auto_variant = false, auto_zchunk = false, auto_order = false;
 };
@@ -55,6 +56,8 @@ extern thread_local int *g_fused_tile_probe;
 bool fused_tile(const Problem &P, int tl, const LaunchCfg &lc, int *tx, int *ty);
 // Output tiles that the fused pass of depth tl has (LaunchCfg::ftile).
 int fused_tiles(const Problem &P, int tl);
+// Whether the pass of depth tl is star7_tb_kernel's (LaunchCfg::halo).
+bool star7_pass(const Problem &P, int tl);
 hipError_t tblock_pass(const Problem &P, int tl, const void *X, const void *Y, void *ZO, void *ZN, const void *src,
                        long long src_idx, const LaunchCfg &lc, hipStream_t st);
 int tb_depths(int kid, int dtype, int *out, int max);

@@ -64,4 +64,39 @@ __device__ __forceinline__ T bload_coef(__amdgpu_buffer_rsrc_t r, unsigned e) {
   }
 }
 
+// f(offset) for every halo cell (outside the interior box) of a field, by the wavefronts
+// 0 .. halo_waves() - 1.  The x-end cells of the interior rows, each on a cache line of its
+// own, are dealt out 64 to a wavefront (with a wavefront per row, 2 lanes busy, a copy cost a
+// call at 389 x 270 x 331 FP32 23 us instead of 18); the rows in the y and z halo get one each.
+template <typename F>
+__device__ __forceinline__ void for_halo_cells(long long w, int lane, int nx, int ny, int nz, int R, long long pitch,
+                                               F &&f) {
+  const int rows = ny + 2 * R;
+  const long long nend = (long long)ny * nz * 2 * R, nendw = (nend + 63) / 64;
+  if (w < nendw) {
+    const long long c = w * 64 + lane, q = c / (2 * R);
+    const int e = (int)(c % (2 * R)), j = (int)(q % ny) + R, k = (int)(q / ny) + R;
+    if (c < nend) f(((long long)k * rows + j) * pitch + (e < R ? e : nx + e));
+    return;
+  }
+  w -= nendw;
+  int j, k;
+  if (w < 2 * R * (long long)rows) {
+    j = (int)(w % rows);
+    k = (int)(w / rows);
+    if (k >= R) k += nz;
+  } else {
+    w -= 2 * R * (long long)rows;
+    j = (int)(w % (2 * R));
+    if (j >= R) j += ny;
+    k = (int)(w / (2 * R)) + R;
+    if (k >= nz + R) return;
+  }
+  const long long o = ((long long)k * rows + j) * pitch;
+  for (int i = lane; i < nx + 2 * R; i += 64) f(o + i);
+}
+inline long long halo_waves(int ny, int nz, int R) {
+  return ((long long)ny * nz * 2 * R + 63) / 64 + 2LL * R * (ny + 2 * R + nz);
+}
+
 }  // namespace gr

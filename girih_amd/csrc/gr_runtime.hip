@@ -30,6 +30,7 @@
 #include "../../include/girih_gpu.h"
 #include "gr_internal.hpp"
 #include "gr_launch.hpp"
+#include "gr_plane.hpp"
 
 namespace {
 
@@ -271,12 +272,12 @@ using namespace gr;
 
 // What a captured step sequence depends on besides the (fixed) field allocations.
 struct GraphKey {
-  int napply, parity, lu0, lu1, variant, zchunk, t_block, xcd_order, ftile, autos, fuse;
+  int napply, parity, lu0, lu1, variant, zchunk, t_block, xcd_order, ftile, autos, fuse, exposed;
   long long napplied;  // -1 unless a source is active (its pointers are baked into the graph)
   bool operator==(const GraphKey &o) const {
     return napply == o.napply && parity == o.parity && lu0 == o.lu0 && lu1 == o.lu1 && variant == o.variant &&
            zchunk == o.zchunk && t_block == o.t_block && xcd_order == o.xcd_order && ftile == o.ftile && autos == o.autos && fuse == o.fuse &&
-           napplied == o.napplied;
+           exposed == o.exposed && napplied == o.napplied;
   }
 };
 
@@ -739,6 +740,7 @@ static int sync_spares(gr_handle *h);
 static int enqueue_apps(gr_handle *h, int napply, bool fuse, int *nlaunch);
 static int finish_step(gr_handle *h, int napply, int launches);
 static bool trades_buffers(const gr_handle *h, int napply);
+static int rest_depth(const gr_handle *h, int rest);
 static void drop_graph(gr_handle *h) {
   if (h->gexec) {
     (void)hipStreamSynchronize(h->stream);  // a replay may still be running
@@ -792,7 +794,8 @@ extern "C" int gr_step(gr_handle *h, int napply) {
     // a third buffer lets the last pass write both levels that a call leaves; without the
     // memory for it a call ends with a single sweep
     if (ensure_spares(h, 1) == GR_OK) {
-      if ((rc = sync_spares(h))) return rc;
+      const bool in_pass = h->exposed && star7_pass(h->P, rest_depth(h, napply));  // enqueue_first_order
+      if (napply > 1 && !in_pass && (rc = sync_spares(h))) return rc;
     } else {
       (void)hipGetLastError();
       h->no_spare = true;
@@ -800,7 +803,8 @@ extern "C" int gr_step(gr_handle *h, int napply) {
   }
   // graph mode: replay the launch sequence of an identical earlier call
   GraphKey key{napply, h->parity, h->lu[0], h->lu[1], h->lc.variant, h->lc.zchunk, h->lc.t_block, h->lc.xcd_order,
-               h->lc.ftile, h->lc.auto_variant + 2 * h->lc.auto_zchunk + 4 * h->lc.auto_order, fuse ? 1 : 0, -1};
+               h->lc.ftile, h->lc.auto_variant + 2 * h->lc.auto_zchunk + 4 * h->lc.auto_order, fuse ? 1 : 0,
+               h->exposed ? 1 : 0, -1};
   if (h->src && h->napplied < h->nsrc) key.napplied = h->napplied;  // source pointers are baked in
   if (h->use_graph && napply > 0 && !(fuse && trades_buffers(h, napply))) {
     if (!(h->gexec && h->gkey == key)) {
@@ -950,6 +954,8 @@ static int enqueue_first_order(gr_handle *h, int napply, int *nlaunch) {
     const void *srcp = has_src ? (const char *)h->src + (size_t)app * es : nullptr;
     const long long sidx = has_src ? h->src_idx : -1;
     LaunchCfg lc = ops[i] > 1 ? fused_cfg(h, ops[i]) : h->lc;
+    // the first pass brings the spare the halo, which the caller may have rewritten
+    if (i == 0 && h->exposed && star7_pass(P, ops[0])) lc.halo = field_base(h, h->fbuf[sp[0]]);
     lc.down = (i & 1) && P.kernel == 5 && z_turns(P);
     const void *in = field_base(h, h->fbuf[x]);
     hipError_t e;
@@ -1525,48 +1531,16 @@ __global__ void init_fields_kernel(T *u1, T *u2, T *r2, int mode, uint64_t seed,
   u2[o] = val;
 }
 
-// f(offset) for every halo cell (outside the interior box) of a field.  The rows in the y
-// and z halo get one wavefront each; the 2R x-end cells of the interior rows, each on a
-// cache line of its own, are dealt out 64 to a wavefront (with a wavefront per row, 2 lanes
-// busy, the copy cost a call at 389 x 270 x 331 FP32 23 us instead of 18).
-template <typename F>
-__device__ __forceinline__ void for_halo_cells(int nx, int ny, int nz, int R, long long pitch, F &&f) {
-  const int rows = ny + 2 * R, lane = threadIdx.x % 64;
-  const long long nend = (long long)ny * nz * 2 * R, nendw = (nend + 63) / 64;
-  long long w = (long long)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
-  if (w < nendw) {
-    const long long c = w * 64 + lane, q = c / (2 * R);
-    const int e = (int)(c % (2 * R)), j = (int)(q % ny) + R, k = (int)(q / ny) + R;
-    if (c < nend) f(((long long)k * rows + j) * pitch + (e < R ? e : nx + e));
-    return;
-  }
-  w -= nendw;
-  int j, k;
-  if (w < 2 * R * (long long)rows) {
-    j = (int)(w % rows);
-    k = (int)(w / rows);
-    if (k >= R) k += nz;
-  } else {
-    w -= 2 * R * (long long)rows;
-    j = (int)(w % (2 * R));
-    if (j >= R) j += ny;
-    k = (int)(w / (2 * R)) + R;
-    if (k >= nz + R) return;
-  }
-  const long long o = ((long long)k * rows + j) * pitch;
-  for (int i = lane; i < nx + 2 * R; i += 64) f(o + i);
-}
-
 // Workgroups of 256 lanes of a kernel over P's halo cells.
-static unsigned halo_blocks(const Problem &P) {
-  const long long waves = ((long long)P.ny * P.nz * 2 * P.R + 63) / 64 + 2LL * P.R * (P.rows + P.nz);
-  return (unsigned)((waves + 3) / 4);
+static unsigned halo_blocks(const Problem &P) { return (unsigned)((halo_waves(P.ny, P.nz, P.R) + 3) / 4); }
+__device__ __forceinline__ long long block_wave() {
+  return (long long)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
 }
 
 // flag = 1 if U1 and U2 differ (bitwise) anywhere outside the interior box
 template <typename U>
 __global__ void halo_diff_kernel(const U *a, const U *b, int nx, int ny, int nz, int R, long long pitch, int *flag) {
-  for_halo_cells(nx, ny, nz, R, pitch, [&](long long o) {
+  for_halo_cells(block_wave(), threadIdx.x % 64, nx, ny, nz, R, pitch, [&](long long o) {
     if (a[o] != b[o]) *flag = 1;
   });
 }
@@ -1574,7 +1548,7 @@ __global__ void halo_diff_kernel(const U *a, const U *b, int nx, int ny, int nz,
 // the halo of src into d0 (and d1 unless null)
 template <typename U>
 __global__ void halo_copy_kernel(const U *src, U *d0, U *d1, int nx, int ny, int nz, int R, long long pitch) {
-  for_halo_cells(nx, ny, nz, R, pitch, [&](long long o) {
+  for_halo_cells(block_wave(), threadIdx.x % 64, nx, ny, nz, R, pitch, [&](long long o) {
     const U v = src[o];
     d0[o] = v;
     if (d1) d1[o] = v;
@@ -1625,8 +1599,8 @@ static int check_halo_equal(gr_handle *h) {
 }
 
 // The spares get the fields' halo, which passes read but never write.  Once per upload or
-// initial state, and at every call of a handle whose field pointers the caller holds (4 us
-// at 128^3 FP64, 14 at 389 x 270 x 331 FP32, 30 at 512^3 FP32).
+// initial state, and at every call of a handle whose field pointers the caller holds (where
+// the call's first pass cannot bring it along: 4 us at 128^3 FP64, 30 at 512^3 FP32).
 static int sync_spares(gr_handle *h) {
   if (h->exposed) h->spares_synced = false;
   if (h->spares_synced) return GR_OK;

@@ -15,7 +15,8 @@ static hipError_t launch_s7(S7Args<T, C> a, hipStream_t st) {
   a.tiles_y = (a.ny + TY - 1) / TY;
   a.zchunk = (a.zchunk <= 0 || a.zchunk > a.nz) ? a.nz : a.zchunk;
   a.nzc = (a.nz + a.zchunk - 1) / a.zchunk;
-  const dim3 grid(a.tiles_x * a.tiles_y * a.nzc);
+  a.nwork = a.tiles_x * a.tiles_y * a.nzc;
+  const dim3 grid(a.nwork + (a.H ? (unsigned)((halo_waves(a.ny, a.nz, 1) + NT / 64 - 1) / (NT / 64)) : 0u));
   const bool gen = a.src_k >= 0 || a.Z1;
   if constexpr (KID == 5) {
     if (a.down) {  // plane k of the arguments is plane nz + 1 - k of the fields
@@ -62,6 +63,8 @@ static S7Args<T, C> s7_args(const Problem &P, const void *Y, void *Z1, void *Z, 
   a.xcd_order = lc.xcd_order;
   a.zchunk = lc.zchunk;
   a.down = lc.down;
+  a.HS = (const T *)Y;
+  a.H = (T *)lc.halo;
   a.src = (const T *)src;
   a.src_k = src_idx < 0 ? -1 : (int)(src_idx / a.sz);
   a.src_off = src_idx < 0 ? 0 : (int)(src_idx % a.sz) + P.xoff;

@@ -305,6 +305,10 @@ static hipError_t tb6_pass(const Problem &P, const void *Y, void *ZN, const void
 
 thread_local int *g_fused_tile_probe = nullptr;
 
+bool star7_pass(const Problem &P, int tl) {
+  return P.kernel == 1 || (P.kernel == 5 && (tl != 6 || (P.flags & GR_COEF_BF16)));
+}
+
 int fused_tiles(const Problem &P, int tl) {
   if (P.kernel == 5) return k5_tiles(P, tl);
   if (P.kernel == 1) {
@@ -337,8 +341,8 @@ hipError_t tblock_pass(const Problem &P, int tl, const void *X, const void *Y, v
     return P.dtype == GR_F64 ? k1_pass_f64(P, tl, Y, ZO, ZN, src, src_idx, lc, st)
                              : k1_pass_f32(P, tl, Y, ZO, ZN, src, src_idx, lc, st);
   if (P.kernel != 5) return hipErrorInvalidValue;
-  if (tl == 6 && !(P.flags & GR_COEF_BF16)) {
-    if (ZO) return hipErrorInvalidValue;  // the call's last pass is a shallower one
+  if (!star7_pass(P, tl)) {
+    if (ZO || lc.halo) return hipErrorInvalidValue;  // it ends no call and copies no halo
     if (P.dtype == GR_F64) return tb6_pass<double>(P, Y, ZN, src, src_idx, lc, st);
     return tb6_pass<float>(P, Y, ZN, src, src_idx, lc, st);
   }

@@ -39,10 +39,11 @@ def _new_halo(rng, u, v, R):
 @pytest.mark.parametrize("kernel,storage,depth", [(1, "f32", 4), (1, "f64", 3), (5, "f64", 4), (5, "f32", 2),
                                                   (5, "bf16", 6), (5, "f32", 6), (0, "f64", 2), (0, "f32", 2)])
 @pytest.mark.parametrize("graph", [False, True])
-def test_rewritten_halos_reach_fused_passes(kernel, storage, depth, graph):
+@pytest.mark.parametrize("n", [(37, 18, 11), (131, 40, 9)])
+def test_rewritten_halos_reach_fused_passes(kernel, storage, depth, graph, n):
     torch = pytest.importorskip("torch")
     dt = np.float64 if storage == "f64" else np.float32
-    nx, ny, nz = 37, 18, 11
+    nx, ny, nz = n
     u, v, roc2, coef = _random_problem(kernel, nx, ny, nz, dt, 77)
     if storage == "bf16":
         coef = _bf16_round(coef)
@@ -55,9 +56,9 @@ def test_rewritten_halos_reach_fused_passes(kernel, storage, depth, graph):
         st.set_graph(graph)
         a = 0
         # one pass (first-order kernels trade a field for the spare), several, a rest of one
-        for n, napply in enumerate((depth, 3 * depth, depth, depth, 2 * depth + 1, 2 * depth)):
+        for call, napply in enumerate((depth, 3 * depth, depth, depth, 2 * depth + 1, 2 * depth)):
             print("halo", kernel, storage, depth, graph, napply, flush=True)
-            if n > 0:
+            if call > 0:
                 _new_halo(rng, u, v, R)
                 for which, f in ((0, u), (1, v)):
                     _view(torch, st, which).copy_(torch.tensor(f[:, :, :nx + 2 * R].copy(), device="cuda"))
