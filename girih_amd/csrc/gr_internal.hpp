@@ -35,7 +35,7 @@ struct LaunchCfg {
 
 int num_tile_variants(int kid, int dtype);
 // lc with its automatic settings replaced by those for a sweep of a box of nx x ny x nz cells.
-LaunchCfg sweep_cfg(int kid, const LaunchCfg &lc, int nx, int ny, int nz);
+LaunchCfg sweep_cfg(int kid, int dtype, const LaunchCfg &lc, int nx, int ny, int nz);
 void tile_of_variant(int kid, int dtype, int variant, int *tx, int *ty);
 
 size_t elem_size(int dtype);

@@ -136,7 +136,9 @@ void tile_of_variant(int kid, int dtype, int variant, int *tx, int *ty) {
 //    32 planes 486 us, 16 500; on 64-wide tiles, more of which fit a CU, 16: 403 x 300 x
 //    219 FP32 119 us, 32 planes 135), 16 for kernel 1 (512^3 FP32 247 us, 32 planes 248, 128
 //    251), 4 where coefficient arrays are streamed (600 x 600 x 300 kernel 5 FP64 4 planes
-//    1490 us, 8 1534, 16 1558; 403 x 300 x 219 kernel 4 384, 405, 419);
+//    1490 us, 8 1534, 16 1558; 403 x 300 x 219 kernel 4 384, 405, 419), but 16 for kernel 4 in FP64,
+//    whose chunks re-read 8 planes, from 200000 cells a plane on (us per four sweeps at 4 / 16
+//    planes: 512 x 512 x 256 6097 / 5839, 700 x 500 x 200 6601 / 6495, 448 x 330 x 260 3516 / 3578);
 //  * tile: 128 x 16 of 1024 lanes (for kernel 0 with the operand prefetch) where it overhangs
 //    the box no further than 64 x 16 does (256^3 kernel 0 FP32 60 us against 62, 512^3
 //    486 against 520; but 320^3 138 against 133) and there is work for 256 of them, or with
@@ -145,7 +147,7 @@ void tile_of_variant(int kid, int dtype, int variant, int *tx, int *ty) {
 //    FP64 384 x 384 x 100 at 64 planes 638 / 468; 64, kernel 5 FP64 250 x 120 x 200 936 / 583);
 //    else 64 x 16 of 512 lanes (64^3 kernel 0 19 us against 22);
 //  * order: XCD bands of tile rows (403 x 300 x 219 kernel 3 157 us, plain runs 164).
-LaunchCfg sweep_cfg(int kid, const LaunchCfg &lc, int nx, int ny, int nz) {
+LaunchCfg sweep_cfg(int kid, int dtype, const LaunchCfg &lc, int nx, int ny, int nz) {
   LaunchCfg c = lc;
   const bool hot = kid == 0 || kid == 1 || kid == 5;  // kernels with tile variants
   if (lc.auto_variant) {
@@ -159,7 +161,8 @@ LaunchCfg sweep_cfg(int kid, const LaunchCfg &lc, int nx, int ny, int nz) {
     int tx = 64, ty = 16;
     tile_of_variant(kid, 0, c.variant, &tx, &ty);
     const long long tiles = (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
-    const int most = kid == 0 ? (tx > 64 ? 32 : 16) : kid == 1 ? 16 : 4;
+    const bool wide4 = kid == 4 && dtype == GR_F64 && (long long)nx * ny >= 200000;
+    const int most = kid == 0 ? (tx > 64 ? 32 : 16) : kid == 1 || wide4 ? 16 : 4;
     c.zchunk = (int)std::min<long long>(most, std::max<long long>(4, tiles * nz / (tx > 64 ? 256 : 512)));
   }
   if (lc.auto_order) c.xcd_order = 2;
@@ -199,7 +202,7 @@ static void turn(SweepArgs<T, C> &a) {
 // One sweep u <- f(v) with the handle's configuration.
 hipError_t sweep_fields(const Problem &P, void *u, const void *v, const void *src, long long src_idx,
                         const LaunchCfg &cfg, hipStream_t st, const void *uold) {
-  const LaunchCfg lc = sweep_cfg(P.kernel, cfg, P.nx, P.ny, P.nz);
+  const LaunchCfg lc = sweep_cfg(P.kernel, P.dtype, cfg, P.nx, P.ny, P.nz);
   const bool down = lc.down && P.kernel != 5 && z_turns(P);
   const bool fast = (P.flags & GR_FAST) != 0;
   const bool rocs = (P.flags & GR_ROC2_SCALAR) != 0;
@@ -1096,7 +1099,7 @@ extern "C" int gr_get_stats(gr_handle *h, gr_stats *out) {
   if (!h || !out) return fail(GR_EINVAL, "gr_get_stats: null argument");
   gr_stats s = h->stats;
   s.t_block = h->lc.t_block;
-  LaunchCfg lc = sweep_cfg(h->P.kernel, h->lc, h->P.nx, h->P.ny, h->P.nz);  // the settings in use
+  LaunchCfg lc = sweep_cfg(h->P.kernel, h->P.dtype, h->lc, h->P.nx, h->P.ny, h->P.nz);  // the settings in use
   if (lc.t_block > 1) {
     const LaunchCfg f = fused_cfg(h, lc.t_block);
     lc.zchunk = f.zchunk;
@@ -1457,7 +1460,7 @@ extern "C" int gr_sweep_dev(int kernel, int dtype, const int shape[3], int xb, i
   g.xb = xb; g.yb = yb; g.zb = zb; g.xe = xe; g.ye = ye; g.ze = ze;
   LaunchCfg lc;
   lc.auto_variant = lc.auto_zchunk = lc.auto_order = true;
-  hipError_t e = sweep_box(P, g, u, v, sweep_cfg(kernel, lc, xe - xb, ye - yb, ze - zb), nullptr);
+  hipError_t e = sweep_box(P, g, u, v, sweep_cfg(kernel, dtype, lc, xe - xb, ye - yb, ze - zb), nullptr);
   if (e != hipSuccess) return fail(GR_EHIP, "gr_sweep_dev: %s", hipGetErrorString(e));
   HIP_TRY(hipStreamSynchronize(nullptr));
   return GR_OK;

@@ -1,5 +1,6 @@
 """The tile of a sweep nobody tuned, under a z chunk of the caller's: 128 wide only where that
-leaves at least 256 workgroups (kernel 0) or 150.  The sweeps equal the CPU oracle's bit for bit (tolerance 0)."""
+leaves at least 256 workgroups (kernel 0) or 150; and kernel 4's own chunks.  The sweeps
+equal the CPU oracle's bit for bit (tolerance 0)."""
 import numpy as np
 import pytest
 
@@ -20,6 +21,13 @@ def test_tile_under_a_given_chunk(kernel):
             st.set_config(zchunk=chunk)
             s = st.stats()
             assert (s["tile_x"], s["zchunk"]) == (128 if wide else 64, chunk), (kernel, n, chunk)
+
+
+def test_kernel4_chunks():
+    for n, dtype, chunk in [((512, 512, 256), gpu.GR_F64, 16), ((512, 512, 256), gpu.GR_F32, 4),
+                            ((448, 330, 100), gpu.GR_F64, 4), ((500, 400, 3), gpu.GR_F64, 4)]:
+        with gpu.Stepper(4, *n, dtype=dtype) as st:
+            assert st.stats()["zchunk"] == chunk, (n, dtype)
 
 
 @pytest.mark.parametrize("kernel", [0, 1, 5])
